@@ -404,6 +404,14 @@ int stride_mlp_xent(const float* d_z, const uint8_t* d_labels, int64_t n, float 
 int stride_mlp_backward(const uint16_t* d_x, int64_t n, const uint16_t* d_wb, const uint16_t* d_h1,
                         const uint16_t* d_h2, const uint16_t* d_dz, uint16_t* d_dh2,
                         uint16_t* d_dh1, float* d_grad, void* stream);
+/* The same with a workspace of *floats float32 (for n rows), which lets the
+ * weight gradients run as slices of the batch, summed in slice order; with a
+ * smaller workspace, or none (stride_mlp_backward), one slice takes them all. */
+int stride_mlp_backward_ws_floats(int64_t n, int64_t* floats);
+int stride_mlp_backward_ws(const uint16_t* d_x, int64_t n, const uint16_t* d_wb,
+                           const uint16_t* d_h1, const uint16_t* d_h2, const uint16_t* d_dz,
+                           uint16_t* d_dh2, uint16_t* d_dh1, float* d_grad, float* d_ws,
+                           int64_t ws_floats, void* stream);
 /* Adam step `step` (>= 1) on the float32 parameters; refreshes d_wb. */
 int stride_mlp_adam(float* d_params, float* d_m, float* d_v, const float* d_grad, uint16_t* d_wb,
                     int64_t n_params, float lr, float beta1, float beta2, float eps, int32_t step,

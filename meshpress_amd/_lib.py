@@ -104,6 +104,8 @@ SIGNATURES = {
     "stride_mlp_forward": (C.c_int, [p, i64, p, p, p, p, p, p]),
     "stride_mlp_xent": (C.c_int, [p, p, i64, C.c_float, p, p, p]),
     "stride_mlp_backward": (C.c_int, [p, i64, p, p, p, p, p, p, p, p]),
+    "stride_mlp_backward_ws_floats": (C.c_int, [i64, P(i64)]),
+    "stride_mlp_backward_ws": (C.c_int, [p, i64, p, p, p, p, p, p, p, p, i64, p]),
     "stride_mlp_adam": (C.c_int, [p, p, p, p, p, i64, C.c_float, C.c_float, C.c_float, C.c_float,
                                   i32, p]),
     "stride_mlp_to_bf16": (C.c_int, [p, i64, p, p]),

@@ -120,9 +120,13 @@ class ProposalMLP:
         n = x.shape[0]
         dh2 = torch.empty((n, N_HID), dtype=torch.bfloat16, device=x.device)
         dh1 = torch.empty((n, N_HID), dtype=torch.bfloat16, device=x.device)
-        _lib.check(self.L.stride_mlp_backward(_lib.ptr(x), n, _lib.ptr(self.wb), _lib.ptr(h1),
-                                              _lib.ptr(h2), _lib.ptr(dz), _lib.ptr(dh2),
-                                              _lib.ptr(dh1), _lib.ptr(self.g), _lib.stream_ptr()))
+        nws = C.c_int64()
+        _lib.check(self.L.stride_mlp_backward_ws_floats(n, C.byref(nws)))
+        ws = torch.empty(nws.value, dtype=torch.float32, device=x.device)
+        _lib.check(self.L.stride_mlp_backward_ws(
+            _lib.ptr(x), n, _lib.ptr(self.wb), _lib.ptr(h1), _lib.ptr(h2), _lib.ptr(dz),
+            _lib.ptr(dh2), _lib.ptr(dh1), _lib.ptr(self.g), _lib.ptr(ws), nws.value,
+            _lib.stream_ptr()))
         return dh2, dh1
 
     def adam(self, lr, beta1=0.9, beta2=0.999, eps=1e-8):

@@ -192,3 +192,62 @@ def test_training_lowers_loss():
     _, cls, _ = net.heads(z)
     acc = (host(cls) == labels[:, 3:]).mean()
     assert acc > 0.3, acc
+
+
+def _misaligned(t):
+    """A copy of t whose data starts one element past a 16-byte boundary."""
+    torch = _t()
+    b = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    b.copy_(t)
+    assert b.data_ptr() % 16
+    return b
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 27, 28, 63, 64, 65, 4097, 16383, 16384, 16401])
+def test_fused_passes_at_tile_edges(n):
+    """The fused passes give the bits of the tiled GEMM layer by layer, from
+    aligned and misaligned operands; the weight gradients, in slices and in
+    one, stay within the error bound of a float32 sum of n products."""
+    from meshpress_amd import _lib
+    torch = _t()
+    L = _lib.lib()
+    net, p, x, labels = _net(n, n)
+    dx = net.features_to_device(x)
+    o1, o2 = LO.N_IN * LO.N_HID, LO.N_IN * LO.N_HID + LO.N_HID * LO.N_HID
+    W1, W2, W3 = net.wb[:o1], net.wb[o1:o2], net.wb[o2:]
+    b = net.p[LO.N_W:]
+
+    def gemm(A, B, N, K, epi, bias=None, mask=None, tb=0):
+        out = torch.empty((n, N), dtype=torch.float32 if epi == 0 else torch.bfloat16, device="cuda")
+        _lib.check(L.stride_mlp_gemm(_lib.ptr(A), K, 0, _lib.ptr(B), K if tb else N, tb, n, N, K, epi,
+                                     _lib.ptr(bias), _lib.ptr(mask), N, _lib.ptr(out) if epi == 0 else None,
+                                     None if epi == 0 else _lib.ptr(out), N, _lib.stream_ptr()))
+        return out
+
+    h1, h2, z = net.forward(dx)
+    g1 = gemm(dx, W1, 128, 32, 1, b[:128])
+    g2 = gemm(g1, W2, 128, 128, 1, b[128:256])
+    assert torch.equal(h1, g1) and torch.equal(h2, g2)
+    assert torch.equal(z, gemm(g2, W3, 176, 128, 0, b[256:]))
+    dz, loss = net.xent(z, torch.from_numpy(labels).to("cuda"), 1.0 / n)
+    dh2, dh1 = net.backward(dx, h1, h2, dz)
+    k2 = gemm(dz, W3, 128, 176, 2, mask=h2, tb=1)
+    assert torch.equal(dh2, k2) and torch.equal(dh1, gemm(k2, W2, 128, 128, 2, mask=h1, tb=1))
+    pairs = [(host(a), host(g)) for a, g in ((dx, dh1), (h1, dh2), (h2, dz))]
+    want = np.concatenate([(a.T @ g).ravel() for a, g in pairs] + [g.sum(0) for _, g in pairs])
+    size = np.concatenate([(np.abs(a).T @ np.abs(g)).ravel() for a, g in pairs]
+                          + [np.abs(g).sum(0) for _, g in pairs])
+    sliced = net.g.clone()
+    assert np.all(np.abs(host(sliced) - want) <= n * 2.0 ** -23 * size)
+    # misaligned operands, one slice (no workspace)
+    mx, m1, m2, mz = (_misaligned(t) for t in (dx, h1, h2, dz))
+    r1, r2 = _misaligned(torch.empty_like(h1)), _misaligned(torch.empty_like(h2))
+    rz = torch.empty_like(z)
+    _lib.check(L.stride_mlp_forward(_lib.ptr(mx), n, _lib.ptr(net.wb), _lib.ptr(net.p), _lib.ptr(r1),
+                                    _lib.ptr(r2), _lib.ptr(rz), _lib.stream_ptr()))
+    assert torch.equal(r1, h1) and torch.equal(r2, h2) and torch.equal(rz, z)
+    _lib.check(L.stride_mlp_backward(_lib.ptr(mx), n, _lib.ptr(net.wb), _lib.ptr(m1), _lib.ptr(m2),
+                                     _lib.ptr(mz), _lib.ptr(r2), _lib.ptr(r1), _lib.ptr(net.g),
+                                     _lib.stream_ptr()))
+    assert torch.equal(r2, dh2) and torch.equal(r1, dh1)
+    assert np.all(np.abs(host(net.g) - want) <= n * 2.0 ** -23 * size)
