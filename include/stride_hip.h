@@ -7,7 +7,7 @@
  * thread.  Device pointers are HIP device memory; `stream` is a hipStream_t
  * (NULL = the default stream).  Handles are not reentrant: one thread at a
  * time per handle; creating handles is thread safe.  The decodes of one
- * handle share its device scratch (the two-pass walk buffer), so they must
+ * handle share its device scratch (the two-pass walk and residual buffers), so they must
  * not overlap on the GPU: issue them on one stream, or order the streams
  * with events.
  *
@@ -129,7 +129,8 @@ int stride_decoder_outputs(stride_decoder* h, float** d_verts, uint32_t** d_tris
  * library's static 32 MiB device array instead of the decoder's own buffers,
  * and the call allocates nothing.  A decode needing more scratch (64 words
  * + n_v + 4 n_meshlets + 8 in mode 4, 64 otherwise) fails with
- * STRIDE_E_UNSUPPORTED.  Every call on a GPU shares that GPU's one array:
+ * STRIDE_E_UNSUPPORTED; one whose residuals (1.5 times the walk) no longer
+ * fit beside the walk decodes them in its axis lanes, more slowly.  Every call on a GPU shares that GPU's one array:
  * calls that overlap on one GPU (other streams, other threads) race. */
 int stride_decode_noalloc(stride_decoder* h, float* d_verts, uint32_t* d_tris, void* stream);
 /* PDLT v5 only: normalised positions (float32 of the float64 reconstruction,

@@ -183,6 +183,9 @@ struct DecodeSet {
   uint32_t* d_walk = nullptr;
   ChainEntry* d_chains = nullptr;         // token chains (tok_chains > 0)
   uint32_t n_chains = 0;
+  ResidChunk* d_rchunks = nullptr;        // residual chunks (null: not usable)
+  uint16_t* d_resid = nullptr;            // decoded residuals, rstride() entries an axis
+  uint32_t rcap = 0, code_lds = 0;        // staged words of a residual wave, LDS of a code group
   uint32_t n_legacy = 0;
   std::vector<uint32_t> l_base;           // first legacy entry of each mesh
   bool ready = false;                     // the launch layout is complete on the device
@@ -205,6 +208,8 @@ struct DecodeSet {
     (void)hipFree(d_tgroups);
     (void)hipFree(d_walk);
     (void)hipFree(d_chains);
+    (void)hipFree(d_rchunks);
+    (void)hipFree(d_resid);
   }
 
   void drop_graphs() {
@@ -281,7 +286,8 @@ struct DecodeSet {
       MeshletScan* d_scan = nullptr;
       HIP_TRY(hipMemcpy(d_tab, tab.data(), sizeof(MeshletEntry) * n_m, hipMemcpyHostToDevice));
       HIP_TRY(hipMalloc(&d_scan, sizeof(MeshletScan) * n_m));
-      hipError_t e1 = launch_scan(d_buf, d_tab, d_mesh, n_m, d_scan, nullptr);
+      HIP_TRY(hipMalloc(&d_rchunks, sizeof(ResidChunk) * kMaxAxisChunks * (size_t)n_m));
+      hipError_t e1 = launch_scan(d_buf, d_tab, d_mesh, n_m, d_scan, d_rchunks, nullptr);
       hipError_t e2 = e1 == hipSuccess ? hipDeviceSynchronize() : e1;
       hipError_t e3 = e2 == hipSuccess
                           ? hipMemcpy(scan.data(), d_scan, sizeof(MeshletScan) * n_m,
@@ -294,6 +300,7 @@ struct DecodeSet {
     v_base.assign(n_meshes + 1, 0);
     t_base.assign(n_meshes + 1, 0);
     uint64_t vt = 0, tt = 0;
+    bool chunks_ok = narrow() && exact32();
     for (int i = 0; i < n_meshes; ++i) {
       uint64_t vo = 0, to = 0;
       v_base[i] = vt;
@@ -319,6 +326,7 @@ struct DecodeSet {
         e.n_local = s.n_local;
         e.n_tris = s.n_tris;
         e.n_strips = s.n_strips | (s.flags & kFlagRawInFifo);
+        chunks_ok &= !(s.flags & kFlagLongSub);
         e.n_kind0 = s.n_kind0;
         e.resid_bit = s.resid_bit;
         for (int k = 0; k < 6; ++k) e.sub_bit[k] = s.sub_bit[k];
@@ -336,6 +344,10 @@ struct DecodeSet {
     HIP_TRY(hipMemcpy(d_mesh, mp.data(), sizeof(MeshParams) * n_meshes, hipMemcpyHostToDevice));
     if (n_m)
       HIP_TRY(hipMemcpy(d_tab, tab.data(), sizeof(MeshletEntry) * n_m, hipMemcpyHostToDevice));
+    if (!chunks_ok) {
+      (void)hipFree(d_rchunks);
+      d_rchunks = nullptr;
+    }
     HIP_TRY(hipMalloc(&d_v_own, 12 * std::max<uint64_t>(n_v, 1)));
     HIP_TRY(hipMalloc(&d_t_own, 12 * std::max<uint64_t>(n_t, 1)));
     // default launch shape (the fastest measured on the 1.3M- and
@@ -382,14 +394,17 @@ struct DecodeSet {
                      : (split ? 4 * ((words + 3) & ~3ull) + 4 * cu : 8 * ((words + 1) / 2) + 8 * cu);
         };
         group_lds = 0;
+        code_lds = 0;
         for (int i = 0; i < n_meshes; ++i) {
           g_base[i] = (uint32_t)groups.size();
           const uint64_t bb = mp[i].blob_byte * 8ull;
           GroupEntry cur{};
           uint64_t codes = 0;
+          uint32_t code_words = 0;   // mode 4: the code arrays alone
           bool open = false;
           auto close = [&]() {
             if (open) {
+              code_lds = std::max(code_lds, 4 * code_words);
               // mode 1: packed codes after the words, in 8-byte units;
               // mode 2: walk/codes blocks after the words, in 4-byte units
               cur.codes_off = split ? ((cur.n_words + 3) & ~3u) : (cur.n_words + 1) / 2;
@@ -409,6 +424,7 @@ struct DecodeSet {
               cur.m1 = j + 1;
               cur.n_words = (uint32_t)(hi - cur.w_lo);
               codes += unit;
+              code_words += split_code_words(e.n_local, nar);
               continue;
             }
             close();
@@ -422,6 +438,7 @@ struct DecodeSet {
             cur.w_lo = (uint32_t)lo;
             cur.n_words = (uint32_t)(hi - lo);
             codes = unit;
+            code_words = split_code_words(e.n_local, nar);
             open = true;
           }
           close();
@@ -548,9 +565,15 @@ struct DecodeSet {
     }
     // walks at 16-byte aligned slots (walk_slot): n_v + 4 words per meshlet,
     // + 8 for the 4-entry reads past the last one
-    if (!d_walk) HIP_TRY(hipMalloc(&d_walk, 4 * (n_v + 4ull * n_m + 8)));
+    if (!d_walk) HIP_TRY(hipMalloc(&d_walk, 4 * walk_words()));
+    if (use_resid() && !d_resid) HIP_TRY(hipMalloc(&d_resid, 6 * rstride()));
     return STRIDE_OK;
   }
+
+  uint64_t walk_words() const { return n_v + 4ull * n_m + 8; }
+  // the residual scratch holds an entry per walk word and axis
+  uint64_t rstride() const { return (walk_words() + 3) & ~3ull; }
+  bool use_resid() const { return cfg.mode == 4 && cfg.tok_chains > 0 && d_rchunks; }
 
   // Chain token waves: consecutive meshlets of one mesh (those the split
   // groups decode) cut into token chains (chain_tokens with k0 =
@@ -559,6 +582,7 @@ struct DecodeSet {
   // final FIFO per chain, 256 first-sighting words).  Replaces tg and tl;
   // the chain-start scan kernel fills d_chains.
   static constexpr uint64_t kChainLds = 49152;
+  static constexpr uint64_t kResidWords = 4096;
   int chain_layout(const std::vector<GroupEntry>& groups, std::vector<GroupEntry>& tg,
                    uint32_t& tl) {
     const int n_meshes = (int)mp.size();
@@ -566,6 +590,7 @@ struct DecodeSet {
     std::vector<uint32_t> cbase(n_m, 0xFFFFFFFFu);
     tg.clear();
     tl = 0;
+    rcap = 0;
     uint32_t nc = 0;
     for (int i = 0; i < n_meshes; ++i) {
       tg_base[i] = (uint32_t)tg.size();
@@ -578,6 +603,10 @@ struct DecodeSet {
         if (open) {
           tg.push_back(cur);
           tl = std::max<uint32_t>(tl, (uint32_t)need(cur.n_words, rec_words));
+          // the words of the wave's residual sections; longer runs than
+          // kResidWords are read from the stream (resid_wave)
+          const uint64_t rw = ((bb + tab[cur.m1 - 1].end_bit) >> 5) + 5 - axis_stage_lo(bb, tab[cur.m0]);
+          if (rw <= kResidWords) rcap = std::max(rcap, (uint32_t)rw);
         }
         open = false;
       };
@@ -639,13 +668,16 @@ struct DecodeSet {
   struct Scratch {
     uint32_t* walk;
     uint32_t* queue;
+    uint16_t* resid;   // null: the axis lanes decode the residuals themselves
   };
-  Scratch own_scratch() const { return Scratch{d_walk, d_queue}; }
+  Scratch own_scratch() const { return Scratch{d_walk, d_queue, use_resid() ? d_resid : nullptr}; }
   // words of scratch a decode takes: 64 for the queue counter, then the
   // walk slots of the two-pass decode (walk_slot: n_v + 4 per meshlet + 8)
-  uint64_t scratch_words() const {
-    return 64ull + (cfg.mode == 4 ? n_v + 4ull * n_m + 8ull : 0ull);
-  }
+  uint64_t scratch_words() const { return 64ull + (cfg.mode == 4 ? walk_words() : 0ull); }
+  // where the residuals start behind them (16-byte aligned), and the words
+  // of a decode that has them
+  uint64_t resid_word() const { return (scratch_words() + 3) & ~3ull; }
+  uint64_t resid_scratch_words() const { return resid_word() + 3 * rstride() / 2; }
 
   GroupLaunch group_args(float* V, uint32_t* T, uint32_t g0, uint32_t g1, uint32_t* flags,
                          uint32_t tg0 = 0, uint32_t tg1 = 0, const Scratch* sc = nullptr) const {
@@ -671,6 +703,11 @@ struct DecodeSet {
     g.walk = two ? S.walk : nullptr;
     g.chains = two ? d_chains : nullptr;
     g.k0 = (uint32_t)cfg.tok_chains;
+    g.rchunks = d_rchunks;
+    g.resid = two ? S.resid : nullptr;
+    g.rstride = rstride();
+    g.rcap = rcap;
+    g.code_lds_bytes = code_lds;
     if (two) g.grid = 0;
     return g;
   }
@@ -683,7 +720,12 @@ struct DecodeSet {
            (uint64_t)n_groups * sizeof(GroupEntry) +
            (two ? (uint64_t)n_tgroups * sizeof(GroupEntry) + (uint64_t)n_chains * sizeof(ChainEntry)
                 : 0ull) +
-           4ull * n_legacy;
+           (use_resid() ? used_chunks() * sizeof(ResidChunk) : 0ull) + 4ull * n_legacy;
+  }
+  uint64_t used_chunks() const {
+    uint64_t n = 0;
+    for (const MeshletEntry& e : tab) n += (e.n_local + kAxisChunk - 1) / kAxisChunk;
+    return n;
   }
 
   // every mesh has at most 16 bits per axis: the split kernels keep uint16 codes
@@ -691,6 +733,15 @@ struct DecodeSet {
     for (const MeshParams& p : mp)
       for (int d = 0; d < 3; ++d)
         if (p.g_bits[d] > 16) return false;
+    return true;
+  }
+
+  // the 32-bit predictor is exact on 16-bit codes for every mesh and axis
+  bool exact32() const {
+    for (const MeshParams& p : mp)
+      for (int d = 0; d < 3; ++d)
+        if (!irlp32_exact(p.pred_n[3 * d], p.pred_n[3 * d + 1], p.pred_n[3 * d + 2], p.pred_K[d]))
+          return false;
     return true;
   }
 
@@ -1045,7 +1096,11 @@ int stride_decode_noalloc(stride_decoder* h, float* d_verts, uint32_t* d_tris, v
   uint32_t* sp = nullptr;
   int rc = scratch_ptr(dev, &sp);
   if (rc) return rc;
-  const DecodeSet::Scratch sc{sp + 64, sp};
+  // a decode whose residuals do not fit the static scratch as well decodes
+  // them in its axis lanes
+  uint16_t* resid = S.use_resid() && S.resid_scratch_words() <= kScratchWords
+                        ? reinterpret_cast<uint16_t*>(sp + S.resid_word()) : nullptr;
+  const DecodeSet::Scratch sc{sp + 64, sp, resid};
   return S.enqueue(d_verts, d_tris, (hipStream_t)stream, 0, (int)S.mp.size(), &sc);
 }
 

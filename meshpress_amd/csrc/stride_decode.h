@@ -64,11 +64,20 @@ struct GroupLaunch {
   // one token lane per meshlet
   const ChainEntry* chains;
   uint32_t k0;
+  // residuals decoded beside the token chains (16-bit codes in a checked
+  // range, irlp32_exact): the chunk table, the residual scratch (rstride
+  // entries an axis), the staged words of a residual wave and the LDS of the
+  // code-chain groups; resid null = the axis lanes decode the codewords
+  const ResidChunk* rchunks;
+  uint16_t* resid;
+  uint64_t rstride;
+  uint32_t rcap;
+  uint32_t code_lds_bytes;
 };
 
 hipError_t launch_group(const GroupLaunch& d, hipStream_t stream);
 hipError_t launch_scan(const uint8_t* buf, const MeshletEntry* seeds, const MeshParams* meshes,
-                       uint32_t n_m, MeshletScan* out, hipStream_t stream);
+                       uint32_t n_m, MeshletScan* out, ResidChunk* chunks, hipStream_t stream);
 hipError_t launch_decode(const DecodeLaunch& d, const DecodeConfig& c, hipStream_t stream);
 hipError_t launch_chain_scan(const uint8_t* buf, const MeshletEntry* tab, const MeshParams* meshes,
                              const uint32_t* cbase, uint32_t n_m, uint32_t k0, ChainEntry* out,

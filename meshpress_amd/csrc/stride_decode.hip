@@ -27,17 +27,40 @@ namespace stride {
 // ---------------------------------------------------------------------------
 // Index pre-pass
 // ---------------------------------------------------------------------------
+// The chunk table of one meshlet: the roots collect in LDS (64 lanes
+// interleaved), the positions go straight to the table.
+struct ChunkSink {
+  static constexpr bool kOn = true;
+  uint32_t* __restrict__ r;       // words r[64 c]
+  ResidChunk* __restrict__ out;
+  __device__ __forceinline__ void clear() {
+    for (int c = 0; c < kMaxAxisChunks; ++c) r[64 * c] = 0u;
+  }
+  __device__ __forceinline__ void entry(uint32_t i, bool root) {
+    if (root) r[64 * ((i >> 5) & 7u)] |= 1u << (i & 31u);
+  }
+  __device__ __forceinline__ uint32_t roots(uint32_t c) const { return r[64 * (c & 7u)]; }
+  __device__ __forceinline__ void pos(uint32_t c, int sub, uint32_t bits) {
+    out[c & 7u].pos[sub] = (uint16_t)bits;
+  }
+};
+
 __global__ void stride_scan_kernel(const uint8_t* __restrict__ buf,
                                    const MeshletEntry* __restrict__ seeds,
                                    const MeshParams* __restrict__ meshes, uint32_t n_m,
-                                   MeshletScan* __restrict__ out) {
+                                   MeshletScan* __restrict__ out,
+                                   ResidChunk* __restrict__ chunks) {
+  __shared__ uint32_t roots[kMaxAxisChunks * 64];
   const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= n_m) return;
   const MeshletEntry e = seeds[m];
   const MeshParams& P = meshes[e.mesh];
   GlobalWords src{reinterpret_cast<const uint32_t*>(buf + P.blob_byte), (e.end_bit + 31u) / 32u + 2u};
   MeshletScan s;
-  scan_meshlet(src, e.start_bit, e.end_bit, P.g_bits, s);
+  ChunkSink sink{roots + threadIdx.x, chunks + (size_t)m * kMaxAxisChunks};
+  sink.clear();
+  scan_meshlet(src, e.start_bit, e.end_bit, P.g_bits, s, sink);
+  for (uint32_t c = 0; c < (uint32_t)kMaxAxisChunks; ++c) sink.out[c].roots = sink.roots(c);
   out[m] = s;
 }
 
@@ -553,13 +576,109 @@ __global__ void stride_chain_scan_kernel(const uint8_t* __restrict__ buf,
 }
 
 
+// Residuals of the meshlets of a token wave, one lane per 32 walk entries
+// and axis (ResidChunk), in walk order: resid[d * rstride + walk_slot + i].
+// The lanes' bits are staged in LDS (rcap words; read from the stream where a
+// wave's run is longer), their 16-bit residuals collect in LDS rows of 17
+// words and leave as 64-byte runs.  Bound by latency: two loops of a handful
+// of roots and at most 32 parallelogram codewords, after three dependent
+// loads; the token waves beside it, in the same launch, run longer.
+constexpr uint32_t kResidRow = 17;   // words a lane: 32 residuals, one word of padding
+
+template <class Src>
+__device__ __forceinline__ void resid_units(const Src& src, uint32_t* __restrict__ rows,
+                                            const MeshletEntry* __restrict__ tab,
+                                            const MeshParams& P, const GroupEntry& G,
+                                            const ResidChunk* __restrict__ chunks,
+                                            uint16_t* __restrict__ resid, uint64_t rstride,
+                                            int lane) {
+  const uint32_t nmesh = G.m1 - G.m0;
+  const uint32_t nl = (uint32_t)lane < nmesh ? tab[G.m0 + (uint32_t)lane].n_local : 0u;
+  uint32_t total = 0;
+  const uint32_t pre = wave_excl_scan(3u * ((nl + kAxisChunk - 1) / kAxisChunk), total);
+  const uint64_t bb = P.blob_byte * 8ull;
+  for (uint32_t u0 = 0; u0 < total; u0 += 64) {
+    const uint32_t u = u0 + (uint32_t)lane;
+    const bool active = u < total;
+    uint32_t j = 0;   // the unit's meshlet: the last one starting at or before it
+    for (uint32_t q = 1; q < nmesh; ++q)
+      j += u >= (uint32_t)__builtin_amdgcn_readlane((int)pre, (int)q) ? 1u : 0u;
+    j = active ? j : 0u;
+    // the shuffle takes every lane: the meshlet's own lane may be idle
+    const uint32_t ju = (uint32_t)__shfl((int)pre, (int)j, 64);
+    const uint32_t rel = active ? u - ju : 0u;
+    const uint32_t c = rel / 3u;
+    const int d = (int)(rel - 3u * c);
+    const uint32_t m = G.m0 + j;
+    const MeshletEntry e = tab[m];
+    const ResidChunk rc = chunks[(size_t)m * kMaxAxisChunks + c];
+    uint16_t* row = reinterpret_cast<uint16_t*>(rows + kResidRow * (uint32_t)lane);
+    auto out = [row](uint32_t i, uint32_t r) { row[i & 31u] = (uint16_t)r; };
+    const bool rice = __all(axis_rice(src, bb, e, P, d));
+    if (active) {
+      if (rice) resid_chunk<true>(src, bb, e, P, rc, c, d, out);
+      else resid_chunk<false>(src, bb, e, P, rc, c, d, out);
+    }
+    // eight lanes a row: pieces of four residuals, up to the entry count
+    // rounded up to four (inside the meshlet's slot)
+    const uint64_t at = ((uint64_t)d * rstride + walk_slot(P, e, m)) / 4 + 8u * c;
+    const uint32_t left = e.n_local - kAxisChunk * c;
+    const uint32_t pieces = active ? ((left < 32u ? left : 32u) + 3u) / 4u : 0u;
+    wave_sync();
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const int p = it * 64 + lane, cu = p >> 3, part = p & 7;
+      const uint64_t dst = ((uint64_t)(uint32_t)__shfl((int)(at >> 32), cu, 64) << 32) |
+                           (uint32_t)__shfl((int)(uint32_t)at, cu, 64);
+      const uint32_t np = (uint32_t)__shfl((int)pieces, cu, 64);
+      const uint32_t* sp = rows + kResidRow * (uint32_t)cu + 2u * (uint32_t)part;
+      const uint2 v{sp[0], sp[1]};
+      if ((uint32_t)part < np) reinterpret_cast<uint2*>(resid)[dst + (uint32_t)part] = v;
+    }
+    wave_sync();
+  }
+}
+
+__device__ __forceinline__ void resid_wave(uint32_t* __restrict__ lds32,
+                                           const uint32_t* __restrict__ words,
+                                           const MeshletEntry* __restrict__ tab,
+                                           const MeshParams* __restrict__ meshes,
+                                           const GroupEntry& G,
+                                           const ResidChunk* __restrict__ chunks, uint32_t rcap,
+                                           uint16_t* __restrict__ resid, uint64_t rstride,
+                                           int lane) {
+  const MeshParams& P = meshes[tab[G.m0].mesh];
+  const uint64_t bb = P.blob_byte * 8ull;
+  uint32_t* rows = lds32 + rcap;
+  // the group's residual sections and the token sections between them are
+  // one run of words
+  const uint64_t lo = axis_stage_lo(bb, tab[G.m0]);
+  const uint64_t n = ((bb + tab[G.m1 - 1].end_bit) >> 5) + 5 - lo;
+  if (n <= rcap) {
+    stage_words(lds32, words, lo, (uint32_t)n, (uint32_t)lane, 64);
+    wave_sync();
+    resid_units(LdsStaged{lds32, lo}, rows, tab, P, G, chunks, resid, rstride, lane);
+  } else {
+    resid_units(BufferWords{words}, rows, tab, P, G, chunks, resid, rstride, lane);
+  }
+}
+
+// Blocks from n_tok on, when chunks is given, decode the residuals of token
+// wave blockIdx.x - n_tok (resid_wave).
 __global__ __launch_bounds__(64) void stride_chain_tokens_kernel(
     const uint8_t* __restrict__ buf, const MeshletEntry* __restrict__ tab,
     const MeshParams* __restrict__ meshes, const GroupEntry* __restrict__ groups,
     const ChainEntry* __restrict__ chains, uint32_t k0, uint32_t* __restrict__ walk_g,
-    uint32_t* __restrict__ T) {
+    uint32_t* __restrict__ T, uint32_t n_tok, const ResidChunk* __restrict__ chunks, uint32_t rcap,
+    uint16_t* __restrict__ resid, uint64_t rstride) {
   extern __shared__ uint32_t lds32[];
   const int lane = threadIdx.x;
+  if (blockIdx.x >= n_tok) {
+    const GroupEntry R = groups[blockIdx.x - n_tok];
+    resid_wave(lds32, reinterpret_cast<const uint32_t*>(buf), tab, meshes, R, chunks, rcap, resid,
+               rstride, lane);
+    return;
+  }
   const GroupEntry G = groups[blockIdx.x];
   const uint32_t* words = reinterpret_cast<const uint32_t*>(buf);
   const uint32_t nmesh = G.m1 - G.m0;
@@ -777,15 +896,61 @@ __global__ __launch_bounds__(64) void stride_axes_kernel(
   }
 }
 
+// The axis pass over decoded residuals (16-bit codes, irlp32_exact, every
+// code checked in range when the layout was made): three lanes per meshlet
+// run the code chains, then the wave dequantises.  A step is the walk entry's
+// addresses, three LDS reads, the prediction and a store, about 25
+// instructions; bound by the latency of that chain through LDS.  With the
+// codeword decode on the chain (stride_axes_kernel) a step is about 70 and the
+// pass took 46.7 us on 10 meshlets, 55.7 us on the 3.9M-triangle heightfield
+// and 123 us on 43,000 meshlets in 256 streams; this one 35 us and 57 us on
+// the latter two, for 9 and 18 us more in the token pass (residual waves).
+// Whole decodes: 63 -> 35, 92 -> 80 and 203 -> 153 us.
+__global__ __launch_bounds__(64) void stride_code_axes_kernel(
+    const MeshletEntry* __restrict__ tab, const MeshParams* __restrict__ meshes,
+    const GroupEntry* __restrict__ groups, const uint32_t* __restrict__ walk_g,
+    const uint16_t* __restrict__ resid, uint64_t rstride, float* __restrict__ V) {
+  extern __shared__ uint32_t lds32[];
+  const int lane = threadIdx.x;
+  const int slot = lane / 3, d = lane - 3 * slot;
+  const GroupEntry G = groups[blockIdx.x];
+  const uint32_t m = G.m0 + (uint32_t)slot;
+  const bool active = slot < kAxisSlots && m < G.m1;
+  const uint32_t nl = active ? tab[m].n_local : 0u;
+  const uint32_t voff = active ? tab[m].v_off : 0u;
+  const uint32_t gmesh = tab[G.m0].mesh;   // a group lies in one mesh
+  const MeshParams& P = meshes[gmesh];
+  uint32_t total = 0;
+  const uint32_t pre0 = wave_excl_scan(d == 0 ? split_code_words(nl, true) : 0u, total);
+  const uint32_t pre = __shfl(pre0, 3 * (lane < 63 ? slot : 0), 64);
+  if (active) {
+    const uint64_t at = ((P.v_base + voff + 3) & ~3ull) + 4ull * m;   // walk_slot
+    CodeChain ax;
+    ax.init(P, d);
+    code_chain(ax, nl, reinterpret_cast<const Walk4*>(walk_g + at),
+               reinterpret_cast<const uint32_t*>(resid + (uint64_t)d * rstride + at),
+               reinterpret_cast<uint16_t*>(lds32 + pre) + split_code_stride(nl, true) * (uint32_t)d);
+  }
+  wave_sync();
+  SplitDequant dq;
+  for (uint32_t j = 0; j < G.m1 - G.m0; ++j) {
+    const uint32_t pj = (uint32_t)__builtin_amdgcn_readlane((int)pre0, (int)(3 * j));
+    dq.meshlet<true>(reinterpret_cast<const uint16_t*>(lds32 + pj),
+                     (uint32_t)__builtin_amdgcn_readlane((int)nl, (int)(3 * j)),
+                     (uint32_t)__builtin_amdgcn_readlane((int)voff, (int)(3 * j)), gmesh, P, V,
+                     lane);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host launchers
 // ---------------------------------------------------------------------------
 hipError_t launch_scan(const uint8_t* buf, const MeshletEntry* seeds, const MeshParams* meshes,
-                       uint32_t n_m, MeshletScan* out, hipStream_t stream) {
+                       uint32_t n_m, MeshletScan* out, ResidChunk* chunks, hipStream_t stream) {
   if (n_m == 0) return hipSuccess;
   const uint32_t tpb = 64;
   hipLaunchKernelGGL(stride_scan_kernel, dim3((n_m + tpb - 1) / tpb), dim3(tpb), 0, stream, buf,
-                     seeds, meshes, n_m, out);
+                     seeds, meshes, n_m, out, chunks);
   return hipGetLastError();
 }
 
@@ -811,9 +976,14 @@ static hipError_t launch_decode_t(const DecodeLaunch& d, hipStream_t stream) {
 hipError_t launch_group(const GroupLaunch& d, hipStream_t stream) {
   if (d.n_groups == 0) return hipSuccess;
   if (d.walk) {   // mode 4: token pass, then the axis pass
+    // residual waves beside the token waves, then the code chains alone
+    const bool pre = d.resid && d.chains && !d.overflow;
     if (d.n_tgroups && d.chains) {
-      hipLaunchKernelGGL(stride_chain_tokens_kernel, dim3(d.n_tgroups), dim3(64), d.tlds_bytes,
-                         stream, d.buf, d.tab, d.meshes, d.tgroups, d.chains, d.k0, d.walk, d.T);
+      const uint32_t rlds = 4 * (d.rcap + 64 * kResidRow);
+      hipLaunchKernelGGL(stride_chain_tokens_kernel, dim3(d.n_tgroups * (pre ? 2u : 1u)), dim3(64),
+                         pre ? std::max(d.tlds_bytes, rlds) : d.tlds_bytes, stream, d.buf, d.tab,
+                         d.meshes, d.tgroups, d.chains, d.k0, d.walk, d.T, d.n_tgroups, d.rchunks,
+                         d.rcap, d.resid, d.rstride);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
     } else if (d.n_tgroups) {
@@ -821,6 +991,11 @@ hipError_t launch_group(const GroupLaunch& d, hipStream_t stream) {
                          d.buf, d.tab, d.meshes, d.tgroups, d.walk, d.T);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
+    }
+    if (pre) {
+      hipLaunchKernelGGL(stride_code_axes_kernel, dim3(d.n_groups), dim3(64), d.code_lds_bytes,
+                         stream, d.tab, d.meshes, d.groups, d.walk, d.resid, d.rstride, d.V);
+      return hipGetLastError();
     }
     // range checks only where a caller collects them (the layout's validation decode)
     if (d.narrow && d.overflow)

@@ -66,6 +66,8 @@ enum : uint32_t {
 // MeshletEntry::n_strips high bits
 constexpr uint32_t kFlagRawInFifo = 1u << 16;  // a raw token names an id already in the FIFO
 constexpr uint32_t kStripMask = 0xFFFFu;
+// MeshletScan::flags only: a residual substream too long for ResidChunk
+constexpr uint32_t kFlagLongSub = 1u << 17;
 
 // A group of consecutive meshlets of one mesh decoded by one wave, one lane
 // per meshlet; its bit range is staged in LDS as one contiguous word run.
@@ -94,6 +96,18 @@ struct ChainEntry {
 static_assert(sizeof(ChainEntry) == 8, "ChainEntry is 8 bytes");
 constexpr int kMaxChains = 16;     // chains per meshlet (4-bit chain index)
 constexpr int kChainMaxLocal = 240;  // placeholders n_local + 0..15 must fit a byte
+
+// Where the residuals of every 32nd walk entry of a meshlet start, recorded
+// by the index pre-pass: residual lanes decode 32 walk entries of one axis
+// each (stride_chain_tokens_kernel).  A meshlet has kMaxAxisChunks entries, of which
+// the first ceil(n_local / 32) are used.
+struct ResidChunk {
+  uint32_t roots;     // bit i: walk entry 32 c + i is a strip root (the anchor or a delta)
+  uint16_t pos[6];    // bits from sub_bit[s] to the chunk's first value of substream s
+};
+static_assert(sizeof(ResidChunk) == 16, "ResidChunk is 16 bytes");
+constexpr int kAxisChunk = 32;
+constexpr int kMaxAxisChunks = 8;
 
 constexpr int kAxisSlots = 21;   // meshlets per wave of the two-pass axis pass (3 lanes each)
 

@@ -1243,12 +1243,140 @@ STRIDE_DEV bool split_axis_g(const Src& words, uint64_t base,
   return ax.good();
 }
 
+// Chunk c of a meshlet of nl walk entries: the entries that take a value of
+// the parallelogram substream (para) or of the delta substream (the roots but
+// the anchor, entry 0).
+STRIDE_DEV uint32_t chunk_values(uint32_t roots, uint32_t c, uint32_t nl, bool para) {
+  const uint32_t left = nl - c * (uint32_t)kAxisChunk;
+  const uint32_t valid = left >= 32u ? ~0u : (1u << left) - 1u;
+  return (para ? ~roots : (c ? roots : roots & ~1u)) & valid;
+}
+STRIDE_DEV uint32_t bit_count(uint32_t x) { return (uint32_t)__builtin_popcount(x); }
+
+// One residual lane: the residuals of walk entries 32 c .. 32 c + 31 of axis
+// d, modulo 2^16 (all that a chain of 16-bit codes needs), to out(i, r) for
+// entry 32 c + i; the anchor's code stands for entry 0's.  RICE: both
+// substreams are Rice coded.
+template <bool RICE, class Src, class Out>
+STRIDE_DEV void resid_chunk(const Src& words, uint64_t base, const MeshletEntry& e,
+                            const MeshParams& P, const ResidChunk& rc, uint32_t c, int d,
+                            Out& out) {
+  const uint32_t gb0 = (uint32_t)P.g_bits[0], gb1 = (uint32_t)P.g_bits[1],
+                 gb2 = (uint32_t)P.g_bits[2];
+  const uint64_t r0 = base + e.resid_bit;
+  const uint64_t tb = r0 + gb0 + gb1 + gb2;
+  const uint32_t TD = bits_at_src(words, tb + 16u * (uint32_t)d, 16);
+  const uint32_t TP = bits_at_src(words, tb + 16u * (uint32_t)(3 + d), 16);
+  if (c == 0)
+    out(0, bits_at_src(words, r0 + (d > 0 ? gb0 : 0u) + (d > 1 ? gb1 : 0u),
+                       pick3(d, gb0, gb1, gb2)));
+  BitStream<Src> sd, sp;
+  sd.init(words, base + pick3(d, e.sub_bit[0], e.sub_bit[1], e.sub_bit[2]) +
+                     pick3(d, rc.pos[0], rc.pos[1], rc.pos[2]));
+  sp.init(words, base + pick3(d, e.sub_bit[3], e.sub_bit[4], e.sub_bit[5]) +
+                     pick3(d, rc.pos[3], rc.pos[4], rc.pos[5]));
+  auto run = [&](BitStream<Src>& s, uint32_t todo, uint32_t T) {
+    const bool eg = (T >> 8) != 1u;
+    const uint32_t egm = eg ? ~0u : 0u;
+    const int k = (int)(T & 31u);
+    while (todo) {
+      const uint32_t i = (uint32_t)__builtin_ctz(todo);
+      todo &= todo - 1u;
+      uint32_t u;
+      const uint32_t len = RICE ? codeword_rice(s.win, k, u) : codeword_win(s.win, egm, k, u);
+      if (len) {
+        s.drop(len);
+        out(i, (u >> 1) ^ (0u - (u & 1u)));
+      } else {
+        out(i, (uint32_t)codeword_s(s, eg, k));
+      }
+    }
+  };
+  run(sd, chunk_values(rc.roots, c, e.n_local, false), TD);
+  run(sp, chunk_values(rc.roots, c, e.n_local, true), TP);
+}
+
+// One axis lane over decoded residuals: the code chain of axis d along the
+// walk, 16-bit codes, irlp32_exact.  Codes and residuals are taken modulo
+// 2^16: the caller has checked (AxisChain, CHECK) that every code of the
+// meshlet lies in [0, 65535], so the low 16 bits are the code.  Entry 0 is a
+// root whose residual is the anchor's code.
+struct CodeChain {
+  int32_t n0, n1, n2, K, rnd;
+  uint32_t prev = 0;
+  STRIDE_DEV void init(const MeshParams& P, int d) {
+    n0 = (int32_t)pick3(d, (uint32_t)P.pred_n[0], (uint32_t)P.pred_n[3], (uint32_t)P.pred_n[6]);
+    n1 = (int32_t)pick3(d, (uint32_t)P.pred_n[1], (uint32_t)P.pred_n[4], (uint32_t)P.pred_n[7]);
+    n2 = (int32_t)pick3(d, (uint32_t)P.pred_n[2], (uint32_t)P.pred_n[5], (uint32_t)P.pred_n[8]);
+    K = (int32_t)pick3(d, (uint32_t)P.pred_K[0], (uint32_t)P.pred_K[1], (uint32_t)P.pred_K[2]);
+    rnd = K > 0 ? (1 << (K - 1)) : 0;
+  }
+  // w: walk entry, r: its residual in the low 16 bits
+  STRIDE_DEV void step(uint32_t w, uint32_t r, uint16_t* __restrict__ codes) {
+    const uint32_t ca = codes[(w >> 8) & 0xFFu], cb = codes[(w >> 16) & 0xFFu],
+                   cc = codes[w >> 24];
+    const uint32_t pred =
+        (uint32_t)irlp24((int32_t)ca, (int32_t)cb, (int32_t)cc, n0, n1, n2, K, rnd);
+    const uint32_t c = (walk_root(w) ? prev : pred) + r;
+    codes[w & 0xFFu] = (uint16_t)c;
+    prev = c;
+  }
+};
+
+// Eight walk entries and their residuals (16-bit pairs).
+struct Walk8 {
+  Walk4 a, b;
+  uint32_t r[4];
+  STRIDE_DEV void load(const Walk4* __restrict__ w, const uint32_t* __restrict__ rr, uint32_t i) {
+    a = w[2 * i];
+    b = w[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = rr[4 * i + q];
+  }
+};
+
+// The chain of a meshlet of n entries: walk slot and residuals in HBM, read
+// eight entries (about a memory round trip of chain steps) ahead.  Reads whole
+// groups of eight, one past the last: up to entry (n / 8 + 1) * 8 + 7.
+STRIDE_DEV void code_chain(CodeChain& ax, uint32_t n, const Walk4* __restrict__ walk,
+                           const uint32_t* __restrict__ resid, uint16_t* __restrict__ codes) {
+  Walk8 cur, nxt;
+  cur.load(walk, resid, 0);
+  uint32_t i = 0;
+  for (; 8 * i + 8 <= n; ++i) {
+    nxt.load(walk, resid, i + 1);
+    ax.step(cur.a.x, cur.r[0], codes);
+    ax.step(cur.a.y, cur.r[0] >> 16, codes);
+    ax.step(cur.a.z, cur.r[1], codes);
+    ax.step(cur.a.w, cur.r[1] >> 16, codes);
+    ax.step(cur.b.x, cur.r[2], codes);
+    ax.step(cur.b.y, cur.r[2] >> 16, codes);
+    ax.step(cur.b.z, cur.r[3], codes);
+    ax.step(cur.b.w, cur.r[3] >> 16, codes);
+    cur = nxt;
+  }
+  const uint32_t left = n - 8 * i;
+  if (left > 0) ax.step(cur.a.x, cur.r[0], codes);
+  if (left > 1) ax.step(cur.a.y, cur.r[0] >> 16, codes);
+  if (left > 2) ax.step(cur.a.z, cur.r[1], codes);
+  if (left > 3) ax.step(cur.a.w, cur.r[1] >> 16, codes);
+  if (left > 4) ax.step(cur.b.x, cur.r[2], codes);
+  if (left > 5) ax.step(cur.b.y, cur.r[2] >> 16, codes);
+  if (left > 6) ax.step(cur.b.z, cur.r[3], codes);
+}
+
 // Index pre-pass for one meshlet (one lane): parses the whole meshlet once,
 // derives the side-table fields the stream does not store, and validates
 // every field against the meshlet's bit range [start, end).
-template <class Src>
+// The chunks' roots and positions (ResidChunk) go to a sink: entry(i, root)
+// for every walk entry, then roots(c) back and pos(c, s, bits) for every chunk
+// c < chunks and substream s.
+struct NoChunks {
+  static constexpr bool kOn = false;
+};
+template <class Src, class Chunks>
 STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const int32_t* g_bits,
-                             MeshletScan& s) {
+                             MeshletScan& s, Chunks& chunks) {
   s = MeshletScan{};
   const uint32_t limit = end - start;
   BitReader<Src> r;
@@ -1293,7 +1421,11 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
     uint32_t p[3] = {0, 0, 0};
     for (int j = 0; j < 3 && err == kScanOk; ++j) {
       if (!token(p[j])) break;
-      if (!seen.test_set(p[j])) { walk++; kind0++; }
+      if (!seen.test_set(p[j])) {
+        if constexpr (Chunks::kOn) chunks.entry(walk, true);
+        walk++;
+        kind0++;
+      }
     }
     for (uint32_t t = 1; t < L && err == kScanOk; ++t) {
       uint32_t ec = r.bits(1);
@@ -1302,7 +1434,10 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
       if (ec == 0) p[0] = p[1];
       p[1] = p[2];
       p[2] = v;
-      if (!seen.test_set(v)) walk++;
+      if (!seen.test_set(v)) {
+        if constexpr (Chunks::kOn) chunks.entry(walk, false);
+        walk++;
+      }
       if (over()) err = kScanErrOverrun;
     }
     if (over()) err = kScanErrOverrun;
@@ -1327,11 +1462,22 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
   for (int j = 0; j < 6 && err == kScanOk; ++j) {
     s.sub_bit[j] = r.pos;
     uint32_t cnt = j < 3 ? n_delta : n_para;
-    if (cnt == 0) continue;
-    if (kk[j] > 24) { err = kScanErrTag; break; }
-    for (uint32_t i = 0; i < cnt; ++i) {
-      uint64_t u = tag[j] == 1 ? r.rice((int)kk[j], limit) : r.exp_golomb((int)kk[j], limit);
-      if (over() || (u >> 32) != 0) { err = kScanErrOverrun; break; }
+    if (cnt != 0 && kk[j] > 24) { err = kScanErrTag; break; }
+    // chunk by chunk: where each starts, then its values
+    const uint32_t nch = Chunks::kOn ? (nl + kAxisChunk - 1) / kAxisChunk : 1u;
+    for (uint32_t c = 0; c < nch && err == kScanOk; ++c) {
+      uint32_t m = cnt;
+      if constexpr (Chunks::kOn) {
+        const uint32_t rel = r.pos - s.sub_bit[j];
+        if (rel > 0xFFFFu) flags |= kFlagLongSub;
+        chunks.pos(c, j, rel & 0xFFFFu);
+        m = chunk_values(chunks.roots(c), c, nl, j >= 3);
+        m = bit_count(m);
+      }
+      for (uint32_t i = 0; i < m; ++i) {
+        uint64_t u = tag[j] == 1 ? r.rice((int)kk[j], limit) : r.exp_golomb((int)kk[j], limit);
+        if (over() || (u >> 32) != 0) { err = kScanErrOverrun; break; }
+      }
     }
   }
   if (err == kScanOk && over()) err = kScanErrOverrun;
@@ -1340,5 +1486,11 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
   s.flags = flags;
 }
 
+template <class Src>
+STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const int32_t* g_bits,
+                             MeshletScan& s) {
+  NoChunks none;
+  scan_meshlet(src, start, end, g_bits, s, none);
+}
 
 }  // namespace stride

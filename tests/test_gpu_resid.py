@@ -1,0 +1,82 @@
+"""The two-pass decode's residual waves on the GPU, bit for bit against the
+oracle, where their routes part: residual runs staged in LDS or read from the
+stream, substreams too long for the chunk table, more units than lanes, 16-bit
+codes and wider ones, predictors outside 32-bit exactness."""
+import numpy as np
+import pytest
+
+from tests.conftest import gpu_available, ribbon
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not gpu_available(), reason="needs a ROCm GPU")]
+
+
+def stream(V, T, bits, k, pred_n=((1, 1, -1),) * 3, pred_K=(0, 0, 0)):
+    """DPR4 bytes with every residual stream coded as Rice(k), or as
+    Exp-Golomb(-k) for negative k."""
+    from meshpress_amd.encoder.prep import header_f32, prepare
+    p = prepare(V, T, precision_error=1.0 / ((1 << bits) - 1.5), precision_mode="bbox_frac")
+    nat = p["native"]
+    pn, pk = np.array(pred_n, np.int64), np.array(pred_K, np.int64)
+    nat.residuals(pn, pk, export=False)
+    tagk = np.tile(np.array([1, k] if k >= 0 else [2, -k], np.uint8), (p["n_meshlets"], 6))
+    return nat.write(header_f32(p), p["g_bits"], pn, pk, tagk)
+
+
+CASES = {
+    # about 150 bits a value: 8,400 words of residuals in a token wave of four
+    "long_runs": (16, 0, {}),
+    "rice": (16, 7, {}),
+    "exp_golomb": (16, -4, {}),
+    "12_bits": (12, 2, {}),
+    "18_bits": (18, 9, {}),                                    # int32 codes
+    "wide_weights": (16, 7, dict(pred_n=((30000, 30000, -30000),) * 3, pred_K=(15, 15, 15))),
+    "shifted": (16, 7, dict(pred_n=((33, 32, -33), (31, 34, -33), (32, 32, -32)), pred_K=(5, 5, 5))),
+}
+
+
+@pytest.mark.parametrize("tune", [dict(), dict(mode=4, group_size=21, lds_bytes=65536, tok_chains=2, tok_group=32),
+                                  dict(mode=4, group_size=3, lds_bytes=8192, tok_chains=16, tok_group=1)],
+                         ids=["default", "wide_waves", "narrow_waves"])
+@pytest.mark.parametrize("case", CASES)
+def test_residual_waves(coracle, case, tune):
+    from meshpress_amd import workloads
+    from meshpress_amd.utils.paradelta_v5_cuda import ParaDeltaV5GpuDecoder
+    bits, k, kw = CASES[case]
+    V, T = workloads.mesh_with_tris("torus", 6000, 3)
+    data = stream(V, T, bits, k, **kw)
+    dec = ParaDeltaV5GpuDecoder(data)
+    if tune:
+        dec.set_tune(**tune)
+    Vo, To = coracle.decode(data)
+    for _ in range(2):
+        Vg, Tg = dec.decode_to_host()
+        assert np.array_equal(Tg.astype(np.int64), To)
+        assert np.array_equal(Vg.view(np.uint32), Vo.view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [2, 3, 15, 16, 17, 31, 32, 33, 128, 1000])
+def test_chunk_edges(coracle, n):
+    """Meshlets of 2 n vertices, around the 32-entry chunks and the
+    8-entry groups of the chain (256 vertices: all eight chunks)."""
+    from meshpress_amd.utils.paradelta_v5_cuda import ParaDeltaV5GpuDecoder
+    V, T = ribbon(n)
+    data = stream(V, T, 12, 3)
+    Vo, To = coracle.decode(data)
+    Vg, Tg = ParaDeltaV5GpuDecoder(data).decode_to_host()
+    assert np.array_equal(Tg.astype(np.int64), To)
+    assert np.array_equal(Vg.view(np.uint32), Vo.view(np.uint32))
+
+
+def test_substreams_past_the_chunk_table(coracle):
+    """Residuals of thousands in unary: substreams past 65,535 bits."""
+    from meshpress_amd import workloads
+    from meshpress_amd.utils.paradelta_v5_cuda import ParaDeltaV5GpuDecoder
+    V, T = workloads.mesh_with_tris("torus", 600, 3)
+    V = V + np.random.default_rng(0).normal(0, 0.02, V.shape)
+    data = stream(V, T, 16, 0)
+    assert len(data) > 3 * 65535 // 8
+    Vo, To = coracle.decode(data)
+    Vg, Tg = ParaDeltaV5GpuDecoder(data).decode_to_host()
+    assert np.array_equal(Tg.astype(np.int64), To)
+    assert np.array_equal(Vg.view(np.uint32), Vo.view(np.uint32))
