@@ -67,6 +67,16 @@ struct BitReader {
     pos += (uint32_t)n;
     return out;
   }
+  // the next 32 bits, and taking n <= 32 of them
+  STRIDE_DEV uint32_t top() {
+    refill();
+    return (uint32_t)(win >> 32);
+  }
+  STRIDE_DEV void take(uint32_t n) {
+    win <<= n;
+    valid -= (int)n;
+    pos += n;
+  }
   // Count zeros before the next '1' and consume the '1'.  Stops counting
   // once the run passes `limit` bits (malformed input); the caller checks
   // pos against the meshlet end.
@@ -265,6 +275,19 @@ struct MtfLite {
   STRIDE_DEV static uint32_t zero_bytes(uint32_t x) {
     const uint32_t low7 = 0x7F7F7F7Fu;
     return ~(((x & low7) + low7) | x | low7);
+  }
+  // One validated token, a hit on FIFO index val (oldest first) or the raw id
+  // val: returns the local id and moves it to the front; found = 1 for a raw
+  // id that was in the FIFO.
+  STRIDE_DEV uint32_t token(uint32_t raw, uint32_t val, uint32_t& found) {
+    uint32_t j = raw ? n : n - 1 - val;
+    const uint32_t v = raw ? val : rank(j & 15u);
+    const int pf = raw ? find(v) : -1;
+    found = pf >= 0 ? 1u : 0u;
+    j = pf >= 0 ? (uint32_t)pf : j;
+    n += raw && j == n && n < 16 ? 1u : 0u;
+    to_front(j, v);
+    return v;
   }
   // rank of v among the n entries, or -1.  Branch-free: the first byte equal
   // to v over all 16 bytes.  Bytes [n, 16) sit above every entry, so the

@@ -27,41 +27,205 @@ namespace stride {
 // ---------------------------------------------------------------------------
 // Index pre-pass
 // ---------------------------------------------------------------------------
-// The chunk table of one meshlet: the roots collect in LDS (64 lanes
-// interleaved), the positions go straight to the table.
-struct ChunkSink {
+// A scan is one serial chain over every token and codeword of a meshlet,
+// bound by that chain's latency, and read through memory it waited for a
+// refill at most steps (1,330 us for 298 meshlets, one lane each).
+//
+// Few meshlets: one wave each, the chain on the wave's scalar unit.
+// Positions, windows and counters are the same in every lane, the stream
+// words sit in two vector registers (one word a lane, the next 64 read
+// ahead), and what a lane of its own would search or shift (the reuse FIFO,
+// the seen set, the chunk table) is spread over the lanes.  A step then waits
+// for no memory: 132 us for 298 meshlets, but each costs 54 us of a SIMD.
+// Many: one lane each, the bits staged in LDS (264 us for 298 meshlets).  The
+// line is where the SIMDs' waves, one after another, take that long.
+constexpr uint32_t kScanWaveMeshlets = 4096;
+
+// Word source: word(i) of the blob for i rising, 0 from n on.
+struct WaveWords {
+  const uint32_t* __restrict__ g;   // little-endian words of the blob
+  uint32_t n, base;                 // lane l holds words base + l and base + 64 + l
+  uint32_t cur, nxt;                // nxt as stored: swapped only when its turn comes
+  __device__ __forceinline__ uint32_t load(uint32_t i) const { return i < n ? g[i] : 0u; }
+  __device__ __forceinline__ void init(const uint32_t* __restrict__ words, uint32_t count,
+                                       uint32_t first) {
+    g = words;
+    n = count;
+    base = first;
+    nxt = load(base + 64u + (threadIdx.x & 63u));
+    cur = __builtin_bswap32(load(base + (threadIdx.x & 63u)));
+  }
+  __device__ __forceinline__ uint32_t operator()(uint32_t i) {
+    if (i - base >= 64u) {
+      cur = __builtin_bswap32(nxt);
+      base += 64u;
+      nxt = load(base + 64u + (threadIdx.x & 63u));
+    }
+    return (uint32_t)__builtin_amdgcn_readlane((int)cur, (int)(i - base));
+  }
+};
+// The newest-first reuse FIFO, rank r in lane r.
+struct WaveFifo {
+  uint32_t e, n;
+  __device__ __forceinline__ void clear() { e = 0u; n = 0u; }
+  // MtfLite::token.  A hit's value sits at its rank, so the search that a raw
+  // id needs gives either's rank, n for an id that is not there.
+  __device__ __forceinline__ uint32_t token(uint32_t raw, uint32_t val, uint32_t& found) {
+    const uint32_t vh = (uint32_t)__builtin_amdgcn_readlane((int)e, (int)((n - 1u - val) & 15u));
+    const uint32_t v = vh ^ ((vh ^ val) & (0u - raw));
+    const uint32_t at = (uint32_t)__ballot(e == v) & ((1u << n) - 1u);   // n <= 16
+    const uint32_t j = (uint32_t)__builtin_ctz(at | (1u << n));
+    found = raw & ((j - n) >> 31);
+    const uint32_t up = (uint32_t)wave_shr1((int)e, (int)v);
+    e = (threadIdx.x & 63u) <= j ? up : e;
+    n = min(max(n, j + 1u), 16u);
+    return v;
+  }
+};
+// 256 local ids, 32 a lane
+struct WaveSeen {
+  uint32_t w;
+  __device__ __forceinline__ uint32_t fresh(uint32_t v) {
+    const uint32_t old = (uint32_t)__builtin_amdgcn_readlane((int)w, (int)((v >> 5) & 7u));
+    w |= (threadIdx.x & 63u) == (v >> 5) ? 1u << (v & 31u) : 0u;
+    return ~(old >> (v & 31u)) & 1u;
+  }
+};
+// The chunk table: chunk c's roots in lane c, position (c, s) in lane 8 c + s,
+// substream s's start in lane s.
+struct WaveChunks {
   static constexpr bool kOn = true;
-  uint32_t* __restrict__ r;       // words r[64 c]
-  ResidChunk* __restrict__ out;
-  __device__ __forceinline__ void clear() {
-    for (int c = 0; c < kMaxAxisChunks; ++c) r[64 * c] = 0u;
+  uint32_t r, p, sb;
+  __device__ __forceinline__ void entry(uint32_t i, uint32_t root) {
+    r |= (threadIdx.x & 63u) == (i >> 5) ? root << (i & 31u) : 0u;
   }
-  __device__ __forceinline__ void entry(uint32_t i, bool root) {
-    if (root) r[64 * ((i >> 5) & 7u)] |= 1u << (i & 31u);
+  __device__ __forceinline__ uint32_t roots(uint32_t c) const {
+    return (uint32_t)__builtin_amdgcn_readlane((int)r, (int)c);
   }
-  __device__ __forceinline__ uint32_t roots(uint32_t c) const { return r[64 * (c & 7u)]; }
-  __device__ __forceinline__ void pos(uint32_t c, int sub, uint32_t bits) {
-    out[c & 7u].pos[sub] = (uint16_t)bits;
+  __device__ __forceinline__ void pos(uint32_t c, int s, uint32_t bits) {
+    p = (threadIdx.x & 63u) == 8u * c + (uint32_t)s ? bits : p;
+  }
+  __device__ __forceinline__ void sub(MeshletScan&, int j, uint32_t bit) {
+    sb = (threadIdx.x & 63u) == (uint32_t)j ? bit : sb;
   }
 };
 
-__global__ void stride_scan_kernel(const uint8_t* __restrict__ buf,
-                                   const MeshletEntry* __restrict__ seeds,
-                                   const MeshParams* __restrict__ meshes, uint32_t n_m,
-                                   MeshletScan* __restrict__ out,
-                                   ResidChunk* __restrict__ chunks) {
-  __shared__ uint32_t roots[kMaxAxisChunks * 64];
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
+constexpr uint32_t kScanWaves = 4;   // meshlets per workgroup
+
+__global__ __launch_bounds__(64 * kScanWaves) void stride_scan_kernel(
+    const uint8_t* __restrict__ buf, const MeshletEntry* __restrict__ seeds,
+    const MeshParams* __restrict__ meshes, uint32_t n_m, MeshletScan* __restrict__ out,
+    ResidChunk* __restrict__ chunks) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t m =
+      blockIdx.x * kScanWaves + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (m >= n_m) return;
+  const uint32_t start = seeds[m].start_bit, end = seeds[m].end_bit;
+  const MeshParams& P = meshes[seeds[m].mesh];
+  WaveWords src;
+  src.init(reinterpret_cast<const uint32_t*>(buf + P.blob_byte), (end + 31u) / 32u + 2u, start >> 5);
+  MeshletScan s;
+  WaveFifo fifo;
+  fifo.clear();
+  WaveSeen seen{0u};
+  WaveChunks sink{0u, 0u, 0u};
+  scan_meshlet(src, start, end, P.g_bits, s, sink, seen, fifo);
+  // ResidChunk: the roots, then six positions of 16 bits
+  ResidChunk* rc = chunks + (size_t)m * kMaxAxisChunks;
+  if (lane < (uint32_t)kMaxAxisChunks) rc[lane].roots = sink.r;
+  if ((lane & 7u) < 6u) rc[lane >> 3].pos[lane & 7u] = (uint16_t)sink.p;
+  if (lane < 6u) out[m].sub_bit[lane] = sink.sb;
+  if (lane == 0) {
+    MeshletScan& o = out[m];
+    o.n_local = s.n_local;
+    o.n_tris = s.n_tris;
+    o.n_strips = s.n_strips;
+    o.n_kind0 = s.n_kind0;
+    o.resid_bit = s.resid_bit;
+    o.end_bit = s.end_bit;
+    o.error = s.error;
+    o.flags = s.flags;
+  }
+}
+
+// The same by lanes: `kScanLanes` consecutive meshlets a wave, their bits
+// staged in LDS where they are one run of at most kScanWords words of one mesh.
+constexpr uint32_t kScanLanes = 32, kScanWords = 8192;
+
+// the chunk table of a lane's meshlet: the roots collect in LDS, the lanes
+// interleaved
+struct LaneChunks {
+  static constexpr bool kOn = true;
+  uint32_t* __restrict__ r;       // words r[kScanLanes c]
+  ResidChunk* __restrict__ out;
+  MeshletScan* __restrict__ scan;
+  __device__ __forceinline__ void entry(uint32_t i, uint32_t root) {
+    if (root) r[kScanLanes * ((i >> 5) & 7u)] |= 1u << (i & 31u);
+  }
+  __device__ __forceinline__ uint32_t roots(uint32_t c) const { return r[kScanLanes * (c & 7u)]; }
+  __device__ __forceinline__ void pos(uint32_t c, int sub, uint32_t bits) {
+    out[c & 7u].pos[sub] = (uint16_t)bits;
+  }
+  __device__ __forceinline__ void sub(MeshletScan&, int j, uint32_t bit) { scan->sub_bit[j] = bit; }
+};
+
+// Stages the run of meshlets [m0, m1); false (and nothing staged) where it is
+// no run of kScanWords.  lo = its first word, absolute.
+__device__ __forceinline__ bool scan_stage(uint32_t* __restrict__ lds, const uint8_t* buf,
+                                           const MeshletEntry* __restrict__ tab,
+                                           const MeshParams* __restrict__ meshes, uint32_t m0,
+                                           uint32_t m1, uint64_t& lo) {
+  const MeshletEntry &a = tab[m0], &b = tab[m1 - 1];
+  const uint64_t base = meshes[a.mesh].blob_byte / 4;
+  lo = base + (a.start_bit >> 5);
+  // a lane reads up to two words past its meshlet
+  const uint64_t n = base + (((uint64_t)b.end_bit + 31) >> 5) + 2 - lo;
+  const bool staged = a.mesh == b.mesh && b.end_bit > a.start_bit && n <= kScanWords;
+  if (staged)
+    stage_words(lds, reinterpret_cast<const uint32_t*>(buf), lo, (uint32_t)n, threadIdx.x, 64);
+  __syncthreads();
+  return staged;
+}
+
+__global__ __launch_bounds__(64) void stride_scan_lanes_kernel(
+    const uint8_t* __restrict__ buf, const MeshletEntry* __restrict__ seeds,
+    const MeshParams* __restrict__ meshes, uint32_t n_m, MeshletScan* __restrict__ out,
+    ResidChunk* __restrict__ chunks) {
+  __shared__ uint32_t words[kScanWords];
+  __shared__ uint32_t sets[16 * kScanLanes];   // seen sets, then roots
+  const uint32_t lane = threadIdx.x, m0 = blockIdx.x * kScanLanes, m = m0 + lane;
+  uint64_t lo = 0;
+  const bool staged = scan_stage(words, buf, seeds, meshes, m0, min(m0 + kScanLanes, n_m), lo);
+  if (lane >= kScanLanes || m >= n_m) return;
   const MeshletEntry e = seeds[m];
   const MeshParams& P = meshes[e.mesh];
-  GlobalWords src{reinterpret_cast<const uint32_t*>(buf + P.blob_byte), (e.end_bit + 31u) / 32u + 2u};
+  const uint32_t n = (e.end_bit + 31u) / 32u + 2u;   // readable words of the blob
   MeshletScan s;
-  ChunkSink sink{roots + threadIdx.x, chunks + (size_t)m * kMaxAxisChunks};
-  sink.clear();
-  scan_meshlet(src, e.start_bit, e.end_bit, P.g_bits, s, sink);
+  MtfLite fifo;
+  fifo.clear();
+  BitSeen seen{sets + lane, kScanLanes};
+  seen.preset(0);
+  LaneChunks sink{sets + 8 * kScanLanes + lane, chunks + (size_t)m * kMaxAxisChunks, out + m};
+  for (int c = 0; c < kMaxAxisChunks; ++c) sink.r[kScanLanes * c] = 0u;
+  // staged: bits counted from the first staged word
+  const uint32_t w0 = staged ? (uint32_t)(lo - P.blob_byte / 4) : 0u, b0 = w0 << 5;
+  if (staged)
+    scan_meshlet(LdsWords{words, n - w0}, e.start_bit - b0, e.end_bit - b0, P.g_bits, s, sink,
+                 seen, fifo);
+  else
+    scan_meshlet(GlobalWords{reinterpret_cast<const uint32_t*>(buf + P.blob_byte), n}, e.start_bit,
+                 e.end_bit, P.g_bits, s, sink, seen, fifo);
   for (uint32_t c = 0; c < (uint32_t)kMaxAxisChunks; ++c) sink.out[c].roots = sink.roots(c);
-  out[m] = s;
+  MeshletScan& o = out[m];
+  o.n_local = s.n_local;
+  o.n_tris = s.n_tris;
+  o.n_strips = s.n_strips;
+  o.n_kind0 = s.n_kind0;
+  o.resid_bit = s.resid_bit + b0;
+  for (int j = 0; j < 6; ++j) o.sub_bit[j] += b0;
+  o.end_bit = s.end_bit + b0;
+  o.error = s.error;
+  o.flags = s.flags;
 }
 
 // ---------------------------------------------------------------------------
@@ -560,21 +724,44 @@ __global__ __launch_bounds__(64) void stride_tokens_kernel(
 // LDS: staged words | records (each meshlet's padded to an even count) |
 // the final FIFO of each chain (16 bytes) | first sightings (256 words).
 // ---------------------------------------------------------------------------
-__global__ void stride_chain_scan_kernel(const uint8_t* __restrict__ buf,
-                                         const MeshletEntry* __restrict__ tab,
-                                         const MeshParams* __restrict__ meshes,
-                                         const uint32_t* __restrict__ cbase, uint32_t n_m,
-                                         uint32_t k0, ChainEntry* __restrict__ out) {
-  const uint32_t m = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64 * kScanWaves) void stride_chain_scan_kernel(
+    const uint8_t* __restrict__ buf, const MeshletEntry* __restrict__ tab,
+    const MeshParams* __restrict__ meshes, const uint32_t* __restrict__ cbase, uint32_t n_m,
+    uint32_t k0, ChainEntry* __restrict__ out) {
+  // one wave per meshlet, as stride_scan_kernel (every lane stores the same)
+  const uint32_t m =
+      blockIdx.x * kScanWaves + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   if (m >= n_m) return;
+  const uint32_t cb = cbase[m];
+  if (cb == 0xFFFFFFFFu) return;
+  const MeshletEntry& e = tab[m];
+  WaveWords src;
+  src.init(reinterpret_cast<const uint32_t*>(buf + meshes[e.mesh].blob_byte),
+           (e.end_bit + 31u) / 32u + 2u, (e.start_bit + 48u) >> 5);
+  chain_starts(src, e.start_bit, e, k0, out + cb);
+}
+
+__global__ __launch_bounds__(64) void stride_chain_scan_lanes_kernel(
+    const uint8_t* __restrict__ buf, const MeshletEntry* __restrict__ tab,
+    const MeshParams* __restrict__ meshes, const uint32_t* __restrict__ cbase, uint32_t n_m,
+    uint32_t k0, ChainEntry* __restrict__ out) {
+  __shared__ uint32_t words[kScanWords];
+  const uint32_t lane = threadIdx.x, m0 = blockIdx.x * kScanLanes, m = m0 + lane;
+  uint64_t lo = 0;
+  const bool staged = scan_stage(words, buf, tab, meshes, m0, min(m0 + kScanLanes, n_m), lo);
+  if (lane >= kScanLanes || m >= n_m) return;
   const uint32_t cb = cbase[m];
   if (cb == 0xFFFFFFFFu) return;
   const MeshletEntry e = tab[m];
   const MeshParams& P = meshes[e.mesh];
-  GlobalWords src{reinterpret_cast<const uint32_t*>(buf + P.blob_byte), (e.end_bit + 31u) / 32u + 2u};
-  chain_starts(src, e.start_bit, e, k0, out + cb);
+  const uint32_t n = (e.end_bit + 31u) / 32u + 2u;
+  const uint32_t w0 = staged ? (uint32_t)(lo - P.blob_byte / 4) : 0u;
+  if (staged)
+    chain_starts(LdsWords{words, n - w0}, e.start_bit - (w0 << 5), e, k0, out + cb);
+  else
+    chain_starts(GlobalWords{reinterpret_cast<const uint32_t*>(buf + P.blob_byte), n}, e.start_bit,
+                 e, k0, out + cb);
 }
-
 
 // Residuals of the meshlets of a token wave, one lane per 32 walk entries
 // and axis (ResidChunk), in walk order: resid[d * rstride + walk_slot + i].
@@ -948,9 +1135,12 @@ __global__ __launch_bounds__(64) void stride_code_axes_kernel(
 hipError_t launch_scan(const uint8_t* buf, const MeshletEntry* seeds, const MeshParams* meshes,
                        uint32_t n_m, MeshletScan* out, ResidChunk* chunks, hipStream_t stream) {
   if (n_m == 0) return hipSuccess;
-  const uint32_t tpb = 64;
-  hipLaunchKernelGGL(stride_scan_kernel, dim3((n_m + tpb - 1) / tpb), dim3(tpb), 0, stream, buf,
-                     seeds, meshes, n_m, out, chunks);
+  if (n_m > kScanWaveMeshlets)
+    hipLaunchKernelGGL(stride_scan_lanes_kernel, dim3((n_m + kScanLanes - 1) / kScanLanes), dim3(64),
+                       0, stream, buf, seeds, meshes, n_m, out, chunks);
+  else
+    hipLaunchKernelGGL(stride_scan_kernel, dim3((n_m + kScanWaves - 1) / kScanWaves),
+                     dim3(64 * kScanWaves), 0, stream, buf, seeds, meshes, n_m, out, chunks);
   return hipGetLastError();
 }
 
@@ -958,9 +1148,12 @@ hipError_t launch_chain_scan(const uint8_t* buf, const MeshletEntry* tab, const 
                              const uint32_t* cbase, uint32_t n_m, uint32_t k0, ChainEntry* out,
                              hipStream_t stream) {
   if (n_m == 0) return hipSuccess;
-  const uint32_t tpb = 64;
-  hipLaunchKernelGGL(stride_chain_scan_kernel, dim3((n_m + tpb - 1) / tpb), dim3(tpb), 0, stream,
-                     buf, tab, meshes, cbase, n_m, k0, out);
+  if (n_m > kScanWaveMeshlets)
+    hipLaunchKernelGGL(stride_chain_scan_lanes_kernel, dim3((n_m + kScanLanes - 1) / kScanLanes),
+                       dim3(64), 0, stream, buf, tab, meshes, cbase, n_m, k0, out);
+  else
+    hipLaunchKernelGGL(stride_chain_scan_kernel, dim3((n_m + kScanWaves - 1) / kScanWaves),
+                     dim3(64 * kScanWaves), 0, stream, buf, tab, meshes, cbase, n_m, k0, out);
   return hipGetLastError();
 }
 

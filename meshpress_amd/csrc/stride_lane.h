@@ -545,35 +545,37 @@ STRIDE_DEV uint32_t chain_end(const ChainEntry& c, uint32_t n_tok, uint32_t lm) 
 // from bit `base`), written to out[0 .. chain_count).  A strip of length 0
 // has three root tokens, as one of length 1 (PDLT v5 allows it; DPR4's
 // pre-pass rejects it).  The stream was validated by the pre-pass.
+// A cut needs the FIFO's fill, not its contents: a meshlet cut more than once
+// has no raw id in its FIFO (chain_tokens), so every raw token adds an entry
+// until the FIFO is full.
 template <class Src>
 STRIDE_DEV void chain_starts_at(const Src& src, uint32_t base, uint32_t tok_bit, uint32_t n_tok,
                                 uint32_t n_local, uint32_t lm, ChainEntry* __restrict__ out) {
   BitReader<Src> r;
   r.init(src, tok_bit);
-  int ib = 1;
+  uint32_t ib = 1;
   while ((1u << ib) < n_local + 1) ++ib;
-  Fifo fifo;
-  fifo.clear();
-  uint32_t j = 0, lp2 = 0, c = 0, next = 0;
+  const uint32_t n_cut = chain_count(n_tok, lm);
+  uint32_t j = 0, lp2 = 0, c = 0, next = 0, fill = 0;
   for (uint32_t t = 0; t < n_tok; ++t) {
     if (t == next) {
       ChainEntry ce;
       ce.pos = (r.pos - base) | (t << 16);
-      ce.state = j | (lp2 << 9) | (fifo.n << 19) | (c << 24);
+      ce.state = j | (lp2 << 9) | (fill << 19) | (c << 24);
       next = chain_end(ce, n_tok, lm);
       out[c++] = ce;
+      if (c == n_cut) return;
     }
     if (j == lp2) {
       const uint32_t L = r.bits(16);
       lp2 = (L ? L : 1u) + 2u;
       j = 0;
     }
-    if (j >= 3) r.bits(1);
-    if (r.bits(1) == 0) {
-      fifo.hit(r.bits(5));
-    } else {
-      fifo.raw(r.bits(ib));
-    }
+    // edge bit (not of a root), flag, id: one window
+    const uint32_t body = (j + 253u) >> 8;   // j >= 3 (j < 259)
+    const uint32_t raw = (r.top() << body) >> 31;
+    fill += raw & ((fill - 16u) >> 31);
+    r.take(body + 1u + 5u + ((ib - 5u) & (0u - raw)));
     ++j;
   }
   if (n_tok == 0) out[0] = ChainEntry{0u, 0u};   // one empty chain
@@ -1369,14 +1371,19 @@ STRIDE_DEV void code_chain(CodeChain& ax, uint32_t n, const Walk4* __restrict__ 
 // derives the side-table fields the stream does not store, and validates
 // every field against the meshlet's bit range [start, end).
 // The chunks' roots and positions (ResidChunk) go to a sink: entry(i, root)
-// for every walk entry, then roots(c) back and pos(c, s, bits) for every chunk
+// for every token (root is 0 unless it is a fresh strip root, walk entry i), then roots(c) back and pos(c, s, bits) for every chunk
 // c < chunks and substream s.
+// sub(s, j, bit): substream j starts at `bit`.
 struct NoChunks {
   static constexpr bool kOn = false;
+  STRIDE_DEV void sub(MeshletScan& s, int j, uint32_t bit) { s.sub_bit[j] = bit; }
 };
-template <class Src, class Chunks>
+// Seen: fresh(v) is true on the first sighting of local id v (BitSeen).
+// Reuse: the newest-first reuse FIFO (MtfLite).  The kernel's are spread over
+// a wave's lanes, everything else here is then the same in every lane.
+template <class Src, class Chunks, class Seen, class Reuse>
 STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const int32_t* g_bits,
-                             MeshletScan& s, Chunks& chunks) {
+                             MeshletScan& s, Chunks& chunks, Seen& seen, Reuse& fifo) {
   s = MeshletScan{};
   const uint32_t limit = end - start;
   BitReader<Src> r;
@@ -1391,56 +1398,48 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
     s.error = kScanErrSize;
     return;
   }
-  int ib = 1;
+  uint32_t ib = 1;
   while ((1u << ib) < nl + 1) ++ib;
-  Fifo fifo;
-  fifo.clear();
-  Seen256 seen;
-  seen.clear();
   uint32_t walk = 0, kind0 = 0, tri_total = 0;
   uint32_t err = kScanOk;
   uint32_t flags = 0;
-  auto token = [&](uint32_t& v) -> bool {
-    uint32_t flag = r.bits(1);
-    if (flag == 0) {
-      uint32_t fi = r.bits(5);
-      if (fi >= fifo.n) { err = kScanErrFifo; return false; }
-      v = fifo.hit(fi);
-    } else {
-      v = r.bits(ib);
-      if (v >= nl) { err = kScanErrIndex; return false; }
-      if (fifo.find(v) >= 0) flags |= kFlagRawInFifo;
-      fifo.raw(v);
+  // one token a trip over all strips: j of the strip's lp tokens are done,
+  // the first three its roots
+  uint32_t st = 0, j = 0, lp = 0;
+  for (;;) {
+    if (j == lp) {
+      if (over()) { err = kScanErrOverrun; break; }
+      if (st == ns) break;
+      const uint32_t L = r.bits(16);
+      ++st;
+      tri_total += L;
+      if (L < 1 || tri_total > nt) { err = kScanErrStrips; break; }
+      lp = L + 2;
+      j = 0;
     }
-    return true;
-  };
-  for (uint32_t st = 0; st < ns && err == kScanOk; ++st) {
-    uint32_t L = r.bits(16);
-    tri_total += L;
-    if (L < 1 || tri_total > nt) { err = kScanErrStrips; break; }
-    uint32_t p[3] = {0, 0, 0};
-    for (int j = 0; j < 3 && err == kScanOk; ++j) {
-      if (!token(p[j])) break;
-      if (!seen.test_set(p[j])) {
-        if constexpr (Chunks::kOn) chunks.entry(walk, true);
-        walk++;
-        kind0++;
-      }
+    // edge bit (not of a root), flag, FIFO index or raw id: one window.
+    // Arithmetic on 0 / 1 instead of selects, which become branches where
+    // the whole wave takes them together.
+    const uint32_t body = (j + 253u) >> 8;   // j >= 3 (j < 259)
+    const uint32_t T = r.top() << body;
+    const uint32_t raw = T >> 31;
+    const uint32_t nb = 5u + ((ib - 5u) & (0u - raw));
+    const uint32_t val = (T << 1) >> (32u - nb);
+    r.take(1u + body + nb);
+    const uint32_t lim = fifo.n + ((nl - fifo.n) & (0u - raw));
+    if (val >= lim) {
+      err = over() ? kScanErrOverrun : raw ? kScanErrIndex : kScanErrFifo;
+      break;
     }
-    for (uint32_t t = 1; t < L && err == kScanOk; ++t) {
-      uint32_t ec = r.bits(1);
-      uint32_t v;
-      if (!token(v)) break;
-      if (ec == 0) p[0] = p[1];
-      p[1] = p[2];
-      p[2] = v;
-      if (!seen.test_set(v)) {
-        if constexpr (Chunks::kOn) chunks.entry(walk, false);
-        walk++;
-      }
-      if (over()) err = kScanErrOverrun;
-    }
-    if (over()) err = kScanErrOverrun;
+    uint32_t found = 0;
+    const uint32_t v = fifo.token(raw, val, found);
+    flags |= found * kFlagRawInFifo;
+    const uint32_t fresh = seen.fresh(v) ? 1u : 0u;
+    if constexpr (Chunks::kOn) chunks.entry(walk, fresh & (body ^ 1u));
+    walk += fresh;
+    kind0 += fresh & (body ^ 1u);
+    if (body && over()) { err = kScanErrOverrun; break; }
+    ++j;
   }
   if (err == kScanOk && tri_total != nt) err = kScanErrStrips;
   if (err == kScanOk && walk != nl) err = kScanErrWalk;
@@ -1453,31 +1452,46 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
   r.bits(g_bits[0]);
   r.bits(g_bits[1]);
   r.bits(g_bits[2]);
-  uint32_t tag[6], kk[6];
+  // the six (tag, k) pairs, k in a byte each
+  uint64_t kks = 0;
+  uint32_t egs = 0;
   for (int j = 0; j < 6; ++j) {
-    tag[j] = r.bits(8);
-    kk[j] = r.bits(8);
+    egs |= r.bits(8) != 1u ? 1u << j : 0u;
+    kks |= (uint64_t)r.bits(8) << (8 * j);
   }
   const uint32_t n_delta = kind0 - 1, n_para = nl - kind0;
   for (int j = 0; j < 6 && err == kScanOk; ++j) {
-    s.sub_bit[j] = r.pos;
+    const uint32_t sub0 = r.pos;
+    const uint32_t kk = (uint32_t)(kks >> (8 * j)) & 0xFFu;
+    const bool eg = (egs >> j) & 1u;
+    const uint32_t egm = 0u - ((egs >> j) & 1u);
+    chunks.sub(s, j, sub0);
     uint32_t cnt = j < 3 ? n_delta : n_para;
-    if (cnt != 0 && kk[j] > 24) { err = kScanErrTag; break; }
+    if (cnt != 0 && kk > 24) { err = kScanErrTag; break; }
     // chunk by chunk: where each starts, then its values
     const uint32_t nch = Chunks::kOn ? (nl + kAxisChunk - 1) / kAxisChunk : 1u;
     for (uint32_t c = 0; c < nch && err == kScanOk; ++c) {
       uint32_t m = cnt;
       if constexpr (Chunks::kOn) {
-        const uint32_t rel = r.pos - s.sub_bit[j];
+        const uint32_t rel = r.pos - sub0;
         if (rel > 0xFFFFu) flags |= kFlagLongSub;
         chunks.pos(c, j, rel & 0xFFFFu);
-        m = chunk_values(chunks.roots(c), c, nl, j >= 3);
-        m = bit_count(m);
+        m = bit_count(chunk_values(chunks.roots(c), c, nl, j >= 3));
       }
       for (uint32_t i = 0; i < m; ++i) {
-        uint64_t u = tag[j] == 1 ? r.rice((int)kk[j], limit) : r.exp_golomb((int)kk[j], limit);
-        if (over() || (u >> 32) != 0) { err = kScanErrOverrun; break; }
+        // a codeword within the window is skipped by its length (its value
+        // then lies below 2^32)
+        const uint32_t T = r.top();
+        const uint32_t q = T ? (uint32_t)__builtin_clz(T) : 32u;
+        const uint32_t len = q + 1 + (q & egm) + kk;
+        if (len <= 32) {
+          r.take(len);
+        } else {
+          const uint64_t u = eg ? r.exp_golomb((int)kk, limit) : r.rice((int)kk, limit);
+          if (over() || (u >> 32) != 0) { err = kScanErrOverrun; break; }
+        }
       }
+      if (over()) err = kScanErrOverrun;
     }
   }
   if (err == kScanOk && over()) err = kScanErrOverrun;
@@ -1486,6 +1500,16 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
   s.flags = flags;
 }
 
+template <class Src, class Chunks>
+STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const int32_t* g_bits,
+                             MeshletScan& s, Chunks& chunks) {
+  uint32_t w[8];
+  BitSeen seen{w};
+  seen.preset(0);
+  MtfLite fifo;
+  fifo.clear();
+  scan_meshlet(src, start, end, g_bits, s, chunks, seen, fifo);
+}
 template <class Src>
 STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const int32_t* g_bits,
                              MeshletScan& s) {

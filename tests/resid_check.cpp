@@ -22,7 +22,8 @@ static uint32_t be32(const uint8_t* p) {
 struct Chunks {
   static constexpr bool kOn = true;
   ResidChunk c[kMaxAxisChunks] = {};
-  void entry(uint32_t i, bool root) { if (root) c[i >> 5].roots |= 1u << (i & 31u); }
+  void sub(MeshletScan& s, int j, uint32_t bit) { s.sub_bit[j] = bit; }
+  void entry(uint32_t i, uint32_t root) { if (root) c[i >> 5].roots |= 1u << (i & 31u); }
   uint32_t roots(uint32_t i) const { return c[i].roots; }
   void pos(uint32_t i, int s, uint32_t bits) { c[i].pos[s] = (uint16_t)bits; }
 };

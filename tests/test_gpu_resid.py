@@ -80,3 +80,26 @@ def test_substreams_past_the_chunk_table(coracle):
     Vg, Tg = ParaDeltaV5GpuDecoder(data).decode_to_host()
     assert np.array_equal(Tg.astype(np.int64), To)
     assert np.array_equal(Vg.view(np.uint32), Vo.view(np.uint32))
+
+
+@pytest.mark.parametrize("meshlets", [4095, 4096, 4097])
+def test_scan_by_waves_and_by_lanes(coracle, meshlets):
+    """The pre-pass of a batch on both sides of the line between a wave and a
+    lane per meshlet: one mesh of many meshlets, then streams of one, so that
+    runs of one mesh and runs across meshes both occur."""
+    import torch
+    from meshpress_amd import workloads
+    from meshpress_amd.batch import BatchDecoder
+    big = stream(*workloads.mesh_with_tris("torus", 300000, 1), 12, 3)
+    one = stream(*ribbon(9), 12, 3)
+    n_big = BatchDecoder([big]).n_meshlets
+    bd = BatchDecoder([big] + [one] * (meshlets - n_big))
+    assert bd.n_meshlets == meshlets
+    v, t = bd.decode()
+    torch.cuda.synchronize()
+    got = bd.split(v.cpu().numpy(), t.cpu().numpy())
+    for i, data in ((0, big), (1, one), (len(got) - 1, one)):
+        Vo, To = coracle.decode(data)
+        assert np.array_equal(got[i][1].astype(np.int64), To)
+        assert np.array_equal(got[i][0].view(np.uint32), Vo.view(np.uint32))
+    assert all(np.array_equal(g[0].view(np.uint32), got[1][0].view(np.uint32)) for g in got[2:])
