@@ -358,6 +358,13 @@ int stride_select_codes(const int32_t* d_vals, const int64_t* d_off, int64_t n_s
  * 0..11 then Exp-Golomb k 0..7); the exhaustive labeller. */
 int stride_stream_costs(const int32_t* d_vals, const int64_t* d_off, int64_t n_streams,
                         int64_t* d_costs, void* stream);
+/* The L1 fit of v by (a, b, c) over n samples, as _fit_irls
+ * (encoder/_irlp_fit.py:239-257): d_out receives the three weights and a flag,
+ * 0 or 1, or 2 where the samples leave the weights undetermined (the caller
+ * then solves it by other means).  d_ws: stride_irls_ws_doubles float64. */
+int stride_irls_ws_doubles(int64_t* doubles);
+int stride_irls_fit(const int32_t* d_a, const int32_t* d_b, const int32_t* d_c,
+                    const int32_t* d_v, int64_t n, double* d_ws, double* d_out, void* stream);
 /* IRLP candidate cost (_cost_seeds_njit, encoder/_irlp_fit.py:120-183): for
  * each of S candidates (n0, n1, n2) with shift K, the sum over meshlets of
  * min over the 20 coders of the parallelogram-residual bits of one axis.

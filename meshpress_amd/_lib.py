@@ -95,6 +95,8 @@ SIGNATURES = {
     "stride_select_codes": (C.c_int, [p, p, i64, p, p, p]),
     "stride_stream_costs": (C.c_int, [p, p, i64, p, p]),
     "stride_irlp_cost": (C.c_int, [p, p, p, p, p, i64, p, i32, i32, p, p]),
+    "stride_irls_ws_doubles": (C.c_int, [P(i64)]),
+    "stride_irls_fit": (C.c_int, [p, p, p, p, i64, p, p, p]),
     "stride_irlp_cost_meshlets": (C.c_int, [p, p, p, p, p, i64, p, i32, i32, p, p]),
     "stride_encoder_features": (C.c_int, [p, i32, p, i64, p]),
     "stride_encoder_para_columns": (C.c_int, [p, p, i64, p, p]),

@@ -11,6 +11,8 @@ control flow (seeds, coordinate descent, early stop) stays on the host.
 """
 from __future__ import annotations
 
+import ctypes as C
+
 import numpy as np
 
 from .. import _lib
@@ -70,6 +72,7 @@ class IrlpCost:
     def __init__(self, a, b, c, v, off):
         torch = _torch()
         self.n_m = len(off) - 1
+        self.n = len(a)
         z = np.zeros(1, np.int32)
         self.a = _dev(a if len(a) else z, torch.int32)
         self.b = _dev(b if len(b) else z, torch.int32)
@@ -89,6 +92,24 @@ class IrlpCost:
             self.n_m, _lib.ptr(d_c), S, int(K), _lib.ptr(d_out), _lib.stream_ptr()))
         self.evals += S
         return d_out[:S].cpu().numpy()
+
+
+    def irls_l1(self):
+        """irls_l1 of the samples on the GPU: the three weights, or None where
+        the samples do not determine them well (or there are none)."""
+        if self.n == 0:
+            return None
+        torch = _torch()
+        L = _lib.lib()
+        nws = C.c_int64()
+        _lib.check(L.stride_irls_ws_doubles(C.byref(nws)))
+        ws = torch.empty(nws.value, dtype=torch.float64, device="cuda")
+        d_out = torch.empty(4, dtype=torch.float64, device="cuda")
+        _lib.check(L.stride_irls_fit(_lib.ptr(self.a), _lib.ptr(self.b), _lib.ptr(self.c),
+                                     _lib.ptr(self.v), self.n, _lib.ptr(ws), _lib.ptr(d_out),
+                                     _lib.stream_ptr()))
+        w = d_out.cpu().numpy()
+        return w[:3] if w[3] < 2 else None
 
 
 class IrlpCostAxes:
@@ -214,9 +235,11 @@ def fit_axis_cols(sub, full, d):
     sub, full: (columns (4, 3, n), offsets) of the subsample and of every
     meshlet.  ((n0, n1, n2) int64, K, bits over all samples, evaluations)."""
     cols, off_s = sub
-    X = np.stack([cols[0, d], cols[1, d], cols[2, d]], axis=1).astype(np.float64)
-    w = irls_l1(X, cols[3, d].astype(np.float64))
     cost = _axis_cost(cols, off_s, d)
+    w = cost.irls_l1()
+    if w is None:
+        X = np.stack([cols[0, d], cols[1, d], cols[2, d]], axis=1).astype(np.float64)
+        w = irls_l1(X, cols[3, d].astype(np.float64))
     K, ns, _ = search_axis(cost, w)
     fcost = _axis_cost(full[0], full[1], d)
     b_fit = int(fcost(np.array(ns)[None], int(K))[0])

@@ -100,3 +100,34 @@ def test_stream_costs(kind):
         else:
             rb = min(min(r), min(e))
         assert (tuple(int(x) for x in tagk[i]), int(bits[i])) == (exp, rb), i
+
+
+@pytest.mark.parametrize("n", [3, 64, 511, 513, 5000, 140001])
+@pytest.mark.parametrize("bits", [12, 16, 24])
+def test_irls_matches_the_host(n, bits):
+    """The GPU's L1 fit against the numpy one: both solve in float64, the
+    host from columns of condition about 2^bits / step."""
+    from meshpress_amd.encoder import search
+    rng = np.random.default_rng(n + bits)
+    top, step = (1 << bits) - 1, (1 << bits) / 200.0
+    c = rng.uniform(0, top, n)
+    a, b = c + rng.normal(0, step, n), c + rng.normal(0, step, n)
+    v = 0.9 * a + 0.8 * b - 0.7 * c + rng.laplace(0, 0.2 * step, n)
+    cols = [np.rint(np.clip(x, 0, top)).astype(np.int32) for x in (a, b, c, v)]
+    w = search.IrlpCost(*cols, np.array([0, n])).irls_l1()
+    X = np.stack(cols[:3], 1).astype(np.float64)
+    host = search.irls_l1(X, cols[3].astype(np.float64))
+    assert w is not None and np.abs(w - host).max() < 1e-9
+
+
+def test_irls_leaves_degenerate_fits_to_the_host():
+    from meshpress_amd.encoder import search
+    n = 1000
+    rng = np.random.default_rng(0)
+    c = rng.integers(0, 4096, n).astype(np.int32)
+    z = np.zeros(n, np.int32)
+    off = np.array([0, n])
+    assert search.IrlpCost(c, c, c, c, off).irls_l1() is None        # a = b = c
+    assert search.IrlpCost(z, z, z, z, off).irls_l1() is None        # all zero
+    assert search.IrlpCost(c + 7, c + 7, c, c, off).irls_l1() is None   # a = b
+    assert search.IrlpCost(z[:0], z[:0], z[:0], z[:0], np.array([0, 0])).irls_l1() is None
