@@ -80,13 +80,13 @@ class BitWriter {
   void put(uint64_t value, int n);           // n <= 64
   void put_rice(uint64_t u, int k);
   void put_eg(uint64_t u, int k);
+  void put_bits(const std::vector<uint8_t>& bytes, uint64_t nbits);   // the first nbits
   uint64_t bit_pos() const { return nbits_; }
   std::vector<uint8_t> finish();
-  std::vector<uint8_t>& bytes() { return buf_; }
  private:
   std::vector<uint8_t> buf_;
   uint64_t acc_ = 0;   // pending bits, right aligned
-  int nacc_ = 0;       // 0..7 pending bits after each put
+  int nacc_ = 0;       // 0..31 pending bits after each put
   uint64_t nbits_ = 0;
 };
 
@@ -165,6 +165,6 @@ int sblb_check(const uint8_t* blob, size_t len, std::string& err);
 
 // tagk: per meshlet 12 bytes: (tag,k) x 3 delta then (tag,k) x 3 para.
 std::vector<uint8_t> write_dup(const Prep& P, const Residuals& R, const Header& H,
-                               const uint8_t* tagk);
+                               const uint8_t* tagk, int n_threads);
 
 }  // namespace stride

@@ -235,12 +235,8 @@ class NativePrep:
 
     def write_v5(self, lin3) -> bytes:
         w = np.ascontiguousarray(np.asarray(lin3, dtype=np.float32).reshape(3))
-        n = C.c_size_t()
-        _lib.check(self._L.stride_encoder_write_v5(self._h, _lib.ptr(w), None, 0, C.byref(n)))
-        out = np.zeros(int(n.value), np.uint8)
-        _lib.check(self._L.stride_encoder_write_v5(self._h, _lib.ptr(w), _lib.ptr(out), len(out),
-                                                   C.byref(n)))
-        return out.tobytes()
+        return self._written(lambda *out: self._L.stride_encoder_write_v5(
+            self._h, _lib.ptr(w), *out))
 
     def write(self, f13, g_bits, pred_n, pred_K, tagk) -> bytes:
         f13 = np.ascontiguousarray(np.asarray(f13, dtype=np.float32).reshape(13))
@@ -248,14 +244,21 @@ class NativePrep:
         pn = np.ascontiguousarray(np.asarray(pred_n, dtype=np.int32).reshape(9))
         pk = np.ascontiguousarray(np.asarray(pred_K, dtype=np.int32).reshape(3))
         tk = np.ascontiguousarray(np.asarray(tagk, dtype=np.uint8).reshape(-1))
+        return self._written(lambda *out: self._L.stride_encoder_write(
+            self._h, _lib.ptr(f13), _lib.ptr(gb), _lib.ptr(pn), _lib.ptr(pk), _lib.ptr(tk), *out))
+
+    def _written(self, write) -> bytes:
+        """What write(out, capacity, length) writes.  A call writes the whole
+        stream, so the first one gets room for any ordinary stream (about 2
+        bytes a triangle at 12 bits, 3.5 at 16); its length is known after."""
         n = C.c_size_t()
-        _lib.check(self._L.stride_encoder_write(self._h, _lib.ptr(f13), _lib.ptr(gb), _lib.ptr(pn),
-                                                _lib.ptr(pk), _lib.ptr(tk), None, 0, C.byref(n)))
-        out = np.zeros(int(n.value), np.uint8)
-        _lib.check(self._L.stride_encoder_write(self._h, _lib.ptr(f13), _lib.ptr(gb), _lib.ptr(pn),
-                                                _lib.ptr(pk), _lib.ptr(tk), _lib.ptr(out), len(out),
-                                                C.byref(n)))
-        return out.tobytes()
+        out = np.empty(8 * self.n_tris_total + 64 * self.n_meshlets + 4096, np.uint8)
+        rc = write(_lib.ptr(out), len(out), C.byref(n))
+        if rc != _lib.STRIDE_OK and n.value > len(out):
+            out = np.empty(int(n.value), np.uint8)
+            rc = write(_lib.ptr(out), len(out), C.byref(n))
+        _lib.check(rc)
+        return out[:int(n.value)].tobytes()
 
 
 def prepare(verts, tris, *, max_verts=256, max_tris=256, precision_error=0.0005,
