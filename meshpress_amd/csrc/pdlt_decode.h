@@ -36,6 +36,13 @@ struct PdltSet {
   ChainEntry* d_chains = nullptr;       // parser state at every token chain's start
   RefChunk* d_rchunks = nullptr;        // boundary-ref chunks of the chain token pass
   uint32_t n_rchunks = 0;
+  // code waves: residual codes decoded beside the token chains (code_waves),
+  // cstride entries an axis, from the chunk table; staged words of a wave
+  CodeChunk* d_cchunks = nullptr;
+  int32_t* d_codes = nullptr;
+  bool code_waves = false;
+  uint32_t ccap = 0;
+  uint64_t cstride() const { return ((uint64_t)(H.n_v - H.n_b) + 4ull * H.n_m + 16 + 3) & ~3ull; }
   uint32_t* d_walk = nullptr;           // two-pass walks (n_v - n_b words)
   uint32_t* d_seen = nullptr;           // two-pass seen sets + walk lengths (kSeenWords per meshlet)
   uint32_t* d_refs = nullptr;           // two-pass boundary refs (n_refs words)

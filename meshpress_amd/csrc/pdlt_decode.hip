@@ -228,6 +228,98 @@ __global__ __launch_bounds__(64) void pdlt_tokens_kernel(
   pdlt_refs_out(lds, G, rb, refs_g, lane);
 }
 
+// The residual codes of a token wave's meshlets, one lane per 32 walk entries
+// and axis (CodeChunk): codes_g[d * cstride + pdlt_slot + i].  As resid_wave
+// of the DPR4 decode; codes are 32 bits.
+constexpr uint32_t kCodeRow = 33;   // words a lane: 32 codes, one word of padding
+
+template <class Src>
+__device__ __forceinline__ void pdlt_code_units(const Src& src, uint32_t* __restrict__ rows,
+                                                const PdltEntry* __restrict__ tab,
+                                                const PdltGroup& G,
+                                                const CodeChunk* __restrict__ chunks, uint32_t n_b,
+                                                int32_t* __restrict__ codes_g, uint64_t cstride,
+                                                int lane) {
+  const uint32_t nmesh = G.m1 - G.m0;
+  const uint32_t ni = (uint32_t)lane < nmesh ? tab[G.m0 + (uint32_t)lane].n_int : 0u;
+  uint32_t total = 0;
+  const uint32_t pre = wave_excl_scan(3u * ((ni + kAxisChunk - 1) / kAxisChunk), total);
+  for (uint32_t u0 = 0; u0 < total; u0 += 64) {
+    const uint32_t u = u0 + (uint32_t)lane;
+    const bool active = u < total;
+    // the unit's meshlet: the last one starting at or before it (one of no
+    // interior vertices has no units, and the next starts where it does)
+    uint32_t j = 0;
+    for (uint32_t q = 1; q < nmesh; ++q)
+      j += u >= (uint32_t)__builtin_amdgcn_readlane((int)pre, (int)q) ? 1u : 0u;
+    const uint32_t ju = (uint32_t)__shfl((int)pre, (int)j, 64);
+    const uint32_t m = G.m0 + j;
+    const PdltEntry e = tab[m];
+    const uint32_t rel = u - ju, c = rel / 3u;
+    const int d = (int)(rel - 3u * c);
+    uint32_t pieces = 0;
+    uint64_t at = 0;
+    if (active) {
+      const CodeChunk cc = chunks[(size_t)m * kMaxAxisChunks + c];
+      uint32_t* row = rows + kCodeRow * (uint32_t)lane;
+      auto out = [row](uint32_t i, uint32_t x) { row[i & 31u] = x; };
+      pdlt_code_chunk(src, e, cc, c, d, out);
+      const uint32_t left = e.n_int - kAxisChunk * c;
+      pieces = ((left < 32u ? left : 32u) + 3u) / 4u;
+      at = ((uint64_t)d * cstride + pdlt_slot(e.int_base, m, n_b)) / 4 + 8u * c;
+    }
+    wave_sync();
+    // eight lanes a row, four codes each
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const int p = it * 64 + lane, cu = p >> 3, part = p & 7;
+      const uint64_t dst = ((uint64_t)(uint32_t)__shfl((int)(at >> 32), cu, 64) << 32) |
+                           (uint32_t)__shfl((int)(uint32_t)at, cu, 64);
+      const uint32_t np = (uint32_t)__shfl((int)pieces, cu, 64);
+      const uint32_t* sp = rows + kCodeRow * (uint32_t)cu + 4u * (uint32_t)part;
+      const uint4 v{sp[0], sp[1], sp[2], sp[3]};
+      if ((uint32_t)part < np) reinterpret_cast<uint4*>(codes_g)[dst + (uint32_t)part] = v;
+    }
+    wave_sync();
+  }
+}
+
+__device__ __forceinline__ void pdlt_code_wave(uint32_t* __restrict__ lds,
+                                               const uint32_t* __restrict__ words,
+                                               const PdltEntry* __restrict__ tab,
+                                               const PdltGroup& G,
+                                               const CodeChunk* __restrict__ chunks, uint32_t ccap,
+                                               uint32_t n_b, int32_t* __restrict__ codes_g,
+                                               uint64_t cstride, int lane) {
+  uint32_t* rows = lds + ccap;
+  const uint64_t lo = pdlt_code_lo(tab[G.m0]);
+  const uint64_t n = pdlt_code_words(tab[G.m0], tab[G.m1 - 1]);
+  if (n <= ccap) {
+    stage_words(lds, words, lo, (uint32_t)n, (uint32_t)lane, 64);
+    wave_sync();
+    pdlt_code_units(LdsStaged{lds, lo}, rows, tab, G, chunks, n_b, codes_g, cstride, lane);
+  } else {
+    pdlt_code_units(BufferWords{words}, rows, tab, G, chunks, n_b, codes_g, cstride, lane);
+  }
+}
+
+// Elements of the boundary table a block of the token launch writes.
+constexpr uint32_t kBndPerBlock = 64 * 16;
+
+// What the code waves' launch adds to the token chains': blocks n_tok ..
+// 2 n_tok - 1 decode codes, those after them write the boundary vertices.
+struct PdltCodeArgs {
+  uint32_t n_tok;
+  const CodeChunk* chunks;     // null: token chains alone, walks at pdlt_walk_off
+  uint32_t ccap;
+  int32_t* codes;
+  uint64_t cstride;
+  const double* bnd;
+  uint64_t n3;                 // boundary coordinates
+  PdltParams P;
+  float* V;
+};
+
 // Two-pass decode, pass 1 with token chains: a wave takes consecutive
 // meshlets (up to 64 chains), whose bits from the first header to the end of
 // the last token section are staged in LDS.  Chunk lanes decode the
@@ -247,10 +339,25 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
     const PdltGroup* __restrict__ groups, const ChainEntry* __restrict__ chains,
     const RefChunk* __restrict__ rchunks, uint32_t k0, uint32_t n_b,
     uint32_t* __restrict__ walk_g, uint32_t* __restrict__ seen_g, uint32_t* __restrict__ refs_g,
-    uint32_t* __restrict__ T) {
+    uint32_t* __restrict__ T, PdltCodeArgs X) {
   extern __shared__ uint64_t lds64[];
   uint32_t* lds = reinterpret_cast<uint32_t*>(lds64);
   const int lane = threadIdx.x;
+  if (blockIdx.x >= X.n_tok) {
+    const uint32_t b = blockIdx.x - X.n_tok;
+    if (b < X.n_tok) {
+      const PdltGroup R = groups[b];
+      pdlt_code_wave(lds, words, tab, R, X.chunks, X.ccap, n_b, X.codes, X.cstride, lane);
+      return;
+    }
+    const uint64_t i0 = (uint64_t)(b - X.n_tok) * kBndPerBlock + (uint32_t)lane;
+#pragma unroll 8
+    for (uint32_t q = 0; q < kBndPerBlock / 64; ++q) {
+      const uint64_t i = i0 + 64u * q;
+      if (i < X.n3) X.V[i] = pdlt_out(pdlt_bnd(X.bnd[i], X.P), X.P, (int)(i % 3));
+    }
+    return;
+  }
   const PdltGroup G = groups[blockIdx.x];
   const uint32_t nmesh = G.m1 - G.m0;
   const uint32_t c0 = G.pad[0], nch = G.pad[1] - G.pad[0];
@@ -352,7 +459,7 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
       const uint32_t g = rf[bx ? x : 0u];
       return bx ? g : ibase + x;
     };
-    uint32_t* wout = walk_g + pdlt_walk_off(ib, m, n_b);
+    uint32_t* wout = walk_g + (X.chunks ? pdlt_slot(ib, m, n_b) : pdlt_walk_off(ib, m, n_b));
     uint32_t* tout = T + 3ull * toff;
     uint32_t wbase = 0, tbase = 0;
     int cv1 = 0, cv2 = 0;
@@ -442,6 +549,59 @@ __global__ __launch_bounds__(64) void pdlt_chain_kernel(
   pdlt_group_tail<R, true>(lds, lds, G, e, active, role, lane, rel, tab, bnd, P, V, refs_g);
 }
 
+// Two-pass decode, pass 2 over decoded codes: a block holds a meshlet's three
+// reconstructions alone; the boundary ones are gathered, three lanes a
+// meshlet run the chains (walk and codes from HBM), the wave writes the
+// interior vertices.  Bound by the latency of the chain through LDS.  With
+// the codeword decode on the chain and the walk, seen set and bits in LDS
+// (pdlt_chain_kernel) the pass took 46.6 us on the 498,000-triangle heightfield
+// (float64) and 49.2 us on the 199,800-triangle sphere (float32).
+template <class R>
+__global__ __launch_bounds__(64) void pdlt_code_chain_kernel(
+    const PdltEntry* __restrict__ tab, const PdltGroup* __restrict__ groups,
+    const double* __restrict__ bnd, PdltParams P, uint32_t n_b, const uint32_t* __restrict__ walk_g,
+    const int32_t* __restrict__ codes_g, uint64_t cstride, const uint32_t* __restrict__ seen_g,
+    const uint32_t* __restrict__ refs_g, float* __restrict__ V) {
+  extern __shared__ uint64_t lds64[];
+  uint32_t* lds = reinterpret_cast<uint32_t*>(lds64);
+  const int lane = threadIdx.x;
+  const int slot = lane & 15, role = lane >> 4;
+  const PdltGroup G = groups[blockIdx.x];
+  const uint32_t m = G.m0 + (uint32_t)slot;
+  const bool active = m < G.m1;
+  PdltEntry e = {};
+  if (active) e = tab[m];
+  const uint32_t nl = e.n_bnd + e.n_int;
+  R* recon = reinterpret_cast<R*>(lds + e.blk_off);
+  const uint32_t n_emit = active ? seen_g[(uint64_t)kSeenWords * m + 8] : 0u;
+  // interior locals that no strip reaches keep position 0
+  if (active && n_emit != e.n_int)
+    for (uint32_t i = (uint32_t)role; i < 3 * e.n_int; i += 4)
+      recon[(i / e.n_int) * nl + e.n_bnd + i % e.n_int] = (R)0;
+  pdlt_gather_group<R>(lds, G, e, lane, refs_g, bnd, P);
+  __syncthreads();
+  if (active && role > 0) {
+    const uint64_t at = pdlt_slot(e.int_base, m, n_b);
+    pdlt_axis_codes<R>(e.n_bnd, P, recon + (uint32_t)(role - 1) * nl,
+                       reinterpret_cast<const Walk4*>(walk_g + at),
+                       reinterpret_cast<const Walk4*>(codes_g + (uint64_t)(role - 1) * cstride + at),
+                       n_emit);
+  }
+  __syncthreads();
+  for (uint32_t j = 0; j < G.m1 - G.m0; ++j) {
+    const uint32_t nbj = (uint32_t)__builtin_amdgcn_readlane((int)e.n_bnd, (int)j);
+    const uint32_t nij = (uint32_t)__builtin_amdgcn_readlane((int)e.n_int, (int)j);
+    const uint32_t boj = (uint32_t)__builtin_amdgcn_readlane((int)e.blk_off, (int)j);
+    const uint32_t ibj = (uint32_t)__builtin_amdgcn_readlane((int)e.int_base, (int)j);
+    const R* rj = reinterpret_cast<const R*>(lds + boj) + nbj;
+    float* vo = V + 3ull * ibj;
+    for (uint32_t t = lane; t < 3 * nij; t += 64) {
+      const uint32_t i = t / 3, d = t - 3 * i;
+      vo[t] = pdlt_out((double)rj[d * (nbj + nij) + i], P, (int)d);
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Host side
 // ---------------------------------------------------------------------------
@@ -465,6 +625,14 @@ PdltSet::~PdltSet() {
   (void)hipFree(d_chains);
   (void)hipFree(d_rchunks);
   (void)hipFree(d_refs);
+  (void)hipFree(d_cchunks);
+  (void)hipFree(d_codes);
+}
+
+static size_t used_chunks(const PdltHost& H) {
+  size_t n = 0;
+  for (const PdltEntry& e : H.tab) n += (e.n_int + kAxisChunk - 1) / kAxisChunk;
+  return n;
 }
 
 size_t PdltSet::side_bytes() const {
@@ -472,7 +640,8 @@ size_t PdltSet::side_bytes() const {
          H.bnd.size() * sizeof(double) +
          (two_pass ? tok_groups.size() * sizeof(PdltGroup) : 0) +
          (two_pass && chain_waves ? n_chains * sizeof(ChainEntry) + n_rchunks * sizeof(RefChunk)
-                                  : 0);
+                                  : 0) +
+         (code_waves ? used_chunks(H) * sizeof(CodeChunk) : 0);
 }
 
 int PdltSet::build(const uint8_t* d, size_t len) {
@@ -481,7 +650,8 @@ int PdltSet::build(const uint8_t* d, size_t len) {
   if (rc) return set_error(rc, err);
   // two-pass scratch: the walks (one word per interior vertex and one per
   // meshlet) and the seen sets with walk lengths
-  const uint64_t n_walk = H.n_v - H.n_b + H.n_m;
+  // (code waves: 16-byte aligned slots and reads past the last one)
+  const uint64_t n_walk = cstride();
   PDLT_HIP(hipMalloc(&d_walk, 4 * std::max<uint64_t>(1, n_walk)));
   PDLT_HIP(hipMalloc(&d_seen, 4ull * kSeenWords * std::max<uint32_t>(1, H.n_m)));
   PDLT_HIP(hipMalloc(&d_refs, 4 * std::max<uint64_t>(1, H.n_refs)));
@@ -492,6 +662,11 @@ int PdltSet::build(const uint8_t* d, size_t len) {
     PDLT_HIP(hipMemcpy(d_bnd, H.bnd.data(), H.bnd.size() * sizeof(double), hipMemcpyHostToDevice));
   }
   if (!H.tab.empty()) PDLT_HIP(hipMalloc(&d_tab, H.tab.size() * sizeof(PdltEntry)));
+  if (!H.chunks.empty()) {
+    PDLT_HIP(hipMalloc(&d_cchunks, H.chunks.size() * sizeof(CodeChunk)));
+    PDLT_HIP(hipMemcpy(d_cchunks, H.chunks.data(), H.chunks.size() * sizeof(CodeChunk),
+                       hipMemcpyHostToDevice));
+  }
   return set_layout(group_size, lds_budget, tok_lds_budget);
 }
 
@@ -500,17 +675,13 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   std::vector<PdltGroup> gr, tg;
   uint32_t lds = 0, tlds = 0;
   std::vector<PdltEntry> tab = H.tab;
-  // the float32 chain keeps three float32 per vertex, the float64 chain three float64
-  // (the chain pass of the two-pass decode reads the refs from HBM; its
-  // blocks keep the refs slot where pdlt_chain_block_refs says so)
-  int rc = pdlt_layout(tab, gs, budget, gr, lds, err, chain32 ? 3u : 6u,
-                       two_pass == 0 || pdlt_chain_block_refs(chain32 != 0));
   // token chains where every meshlet fits a chain token wave, else the
   // token lanes
   std::vector<ChainEntry> ch;
   std::vector<RefChunk> rch;
   bool cw = false;
-  if (!rc && tok_chains > 0) {
+  int rc = STRIDE_OK;
+  if (tok_chains > 0) {
     rc = pdlt_layout_chains(tab, H.words, tok_chains, tok_group, tg, ch, rch, tlds, err);
     cw = rc == STRIDE_OK;
     if (rc == STRIDE_E_UNSUPPORTED) rc = STRIDE_OK;
@@ -518,7 +689,23 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   // (token lanes in place of chains take 64 meshlets a wave)
   if (!rc && !cw)
     rc = pdlt_layout_tokens(tab, tok_budget, tok_chains > 0 ? 64 : tok_group, tg, tlds, err);
+  // with token chains the residual codes are decoded beside them, where the
+  // chunk table holds every position
+  const bool codes = two_pass && cw && d_cchunks;
+  uint32_t cap = 0;
+  if (codes)
+    for (const PdltGroup& g : tg) {
+      const uint64_t n = pdlt_code_words(tab[g.m0], tab[g.m1 - 1]);
+      if (n <= kCodeWords) cap = std::max(cap, (uint32_t)n);
+    }
+  // the float32 chain keeps three float32 per vertex, the float64 chain three
+  // float64 (the chain pass of the two-pass decode reads the refs from HBM;
+  // its blocks keep the refs slot where pdlt_chain_block_refs says so)
+  if (!rc)
+    rc = pdlt_layout(tab, gs, budget, gr, lds, err, chain32 ? 3u : 6u,
+                     two_pass == 0 || pdlt_chain_block_refs(chain32 != 0), codes);
   if (rc) return set_error(rc, err);
+  if (codes && !d_codes) PDLT_HIP(hipMalloc(&d_codes, 12 * cstride()));
   // the new device tables are built aside and take over only once every
   // allocation and copy has succeeded; until then the set is not ready
   ready = false;
@@ -573,6 +760,8 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   d_chains = nc;
   d_rchunks = nr;
   chain_waves = cw;
+  code_waves = codes;
+  ccap = cap;
   n_chains = (uint32_t)ch.size();
   n_rchunks = (uint32_t)rch.size();
   layout_two_pass = two_pass;
@@ -595,8 +784,36 @@ int PdltSet::decode(float* V, uint32_t* T, int world, hipStream_t s) {
   PdltParams p = H.params;
   p.world = world ? 1 : 0;
   p.chain32 = chain32;
+  const uint64_t n3 = 3ull * H.n_b;
+  PdltCodeArgs x{};
+  x.n_tok = (uint32_t)tok_groups.size();
+  if (!groups.empty() && code_waves) {
+    x.chunks = d_cchunks;
+    x.ccap = ccap;
+    x.codes = d_codes;
+    x.cstride = cstride();
+    x.bnd = d_bnd;
+    x.n3 = n3;
+    x.P = p;
+    x.V = V;
+    const uint32_t bb = (uint32_t)((n3 + kBndPerBlock - 1) / kBndPerBlock);
+    hipLaunchKernelGGL(pdlt_chain_tokens_kernel, dim3(2 * x.n_tok + bb), dim3(64),
+                       std::max(tok_lds_bytes, 4 * (ccap + 64 * kCodeRow)), s, d_words, d_tab,
+                       d_tok_groups, d_chains, d_rchunks, (uint32_t)tok_chains, H.n_b, d_walk,
+                       d_seen, d_refs, T, x);
+    PDLT_HIP(hipGetLastError());
+    if (chain32)
+      hipLaunchKernelGGL(pdlt_code_chain_kernel<float>, dim3((uint32_t)groups.size()), dim3(64),
+                         lds_bytes, s, d_tab, d_groups, d_bnd, p, H.n_b, d_walk, d_codes, x.cstride,
+                         d_seen, d_refs, V);
+    else
+      hipLaunchKernelGGL(pdlt_code_chain_kernel<double>, dim3((uint32_t)groups.size()), dim3(64),
+                         lds_bytes, s, d_tab, d_groups, d_bnd, p, H.n_b, d_walk, d_codes, x.cstride,
+                         d_seen, d_refs, V);
+    PDLT_HIP(hipGetLastError());
+    return STRIDE_OK;
+  }
   if (H.n_b) {
-    const uint64_t n3 = 3ull * H.n_b;
     const uint32_t grid = (uint32_t)std::min<uint64_t>((n3 + 255) / 256, 8192);
     hipLaunchKernelGGL(pdlt_boundary_kernel, dim3(grid), dim3(256), 0, s, d_bnd, n3, p, V);
     PDLT_HIP(hipGetLastError());
@@ -606,7 +823,7 @@ int PdltSet::decode(float* V, uint32_t* T, int world, hipStream_t s) {
     if (chain_waves)
       hipLaunchKernelGGL(pdlt_chain_tokens_kernel, dim3((uint32_t)tok_groups.size()), dim3(64),
                          tok_lds_bytes, s, d_words, d_tab, d_tok_groups, d_chains, d_rchunks,
-                         (uint32_t)tok_chains, H.n_b, d_walk, d_seen, d_refs, T);
+                         (uint32_t)tok_chains, H.n_b, d_walk, d_seen, d_refs, T, x);
     else
       hipLaunchKernelGGL(pdlt_tokens_kernel, dim3((uint32_t)tok_groups.size()), dim3(64),
                          tok_lds_bytes, s, d_words, d_tab, d_tok_groups, H.n_b, d_walk, d_seen,

@@ -29,6 +29,7 @@ struct PdltHost {
   std::vector<uint32_t> words;          // the stream as little-endian words, zero padded
   std::vector<double> bnd;              // boundary table, normalised f64 (n_b x 3)
   std::vector<PdltEntry> tab;
+  std::vector<CodeChunk> chunks;        // kMaxAxisChunks a meshlet; empty when one has no entry
   PdltParams params{};
 };
 
@@ -179,13 +180,15 @@ inline int pdlt_parse(const uint8_t* d, size_t len, PdltHost& H, std::string& er
 
   // pre-pass (the parse of paradelta_v5.py:345-446)
   H.tab.assign(n_m, PdltEntry{});
+  H.chunks.assign((size_t)n_m * kMaxAxisChunks, CodeChunk{});
   std::vector<uint32_t> status(n_m, 0);
   par_for(n_m, [&](int64_t m) {
     if (off[m] >= end_all) {
       status[m] = kV5ErrOverrun;
       return;
     }
-    status[m] = pdlt_scan(src, off[m], end_all, n_b, H.tab[m]);
+    status[m] = pdlt_scan(src, off[m], end_all, n_b, H.tab[m],
+                          H.chunks.data() + (size_t)m * kMaxAxisChunks);
   });
   uint64_t iv = n_b, tv = 0, rv = 0;
   for (uint32_t m = 0; m < n_m; ++m) {
@@ -205,6 +208,11 @@ inline int pdlt_parse(const uint8_t* d, size_t len, PdltHost& H, std::string& er
       return STRIDE_E_UNSUPPORTED;
     }
   }
+  for (uint32_t m = 0; m < n_m; ++m)
+    if (H.chunks[(size_t)m * kMaxAxisChunks].bad) {
+      H.chunks.clear();
+      break;
+    }
   H.n_v = iv;
   H.n_t = tv;
   H.n_refs = rv;
@@ -223,9 +231,11 @@ inline int pdlt_parse(const uint8_t* d, size_t len, PdltHost& H, std::string& er
 // the blocks hold a slot of n_bnd words for the boundary refs (the
 // one-kernel decode decodes them there; the chain pass of the two-pass
 // decode reads them from HBM and keeps the slot only where
-// pdlt_chain_block_refs says so).
+// pdlt_chain_block_refs says so).  codes: the groups' chains take decoded
+// codes, so they stage nothing and a block is its reconstructions alone.
 inline int pdlt_layout(std::vector<PdltEntry>& tab, int gs, int budget, std::vector<PdltGroup>& groups,
-                       uint32_t& lds, std::string& err, uint32_t rw = 6, bool refs = true) {
+                       uint32_t& lds, std::string& err, uint32_t rw = 6, bool refs = true,
+                       bool codes = false) {
   if (gs < 1 || gs > 16) { err = "group_size must be in [1, 16]"; return STRIDE_E_ARG; }
   if (budget < 4096 || budget > 65536) { err = "lds_bytes must be in [4096, 65536]"; return STRIDE_E_ARG; }
   groups.clear();
@@ -240,8 +250,9 @@ inline int pdlt_layout(std::vector<PdltEntry>& tab, int gs, int budget, std::vec
     while (j < n_m && (int)(j - m) < gs) {
       // the words holding [start, end) plus the axis lanes' read-ahead (the
       // stream window reads up to 3 words past its position), even count
-      const uint32_t w = ((((tab[j].end_bit - 1) >> 5) + 6 - g.w_lo) + 1) & ~1u;
-      const uint32_t b = pdlt_block_words(tab[j].n_bnd, tab[j].n_int, rw, refs);
+      const uint32_t w = codes ? 0u : ((((tab[j].end_bit - 1) >> 5) + 6 - g.w_lo) + 1) & ~1u;
+      const uint32_t b = codes ? (rw * (tab[j].n_bnd + tab[j].n_int) + 1) & ~1u
+                               : pdlt_block_words(tab[j].n_bnd, tab[j].n_int, rw, refs);
       if (j > m && 4ull * (w + blk + b) > (uint64_t)budget) break;
       tab[j].blk_off = blk;
       blk += b;

@@ -78,6 +78,20 @@ STRIDE_DEV uint64_t pdlt_walk_off(uint32_t int_base, uint32_t m, uint32_t n_boun
   return (uint64_t)(int_base - n_boundary) + m;
 }
 
+// The decode with code waves: walks and codes at 16-byte aligned slots, with
+// at least n_int entries rounded up to four each (as walk_slot).
+STRIDE_DEV uint64_t pdlt_slot(uint32_t int_base, uint32_t m, uint32_t n_boundary) {
+  return (((uint64_t)(int_base - n_boundary) + 3) & ~3ull) + 4ull * m;
+}
+
+// Where the residual codes of every 32nd walk entry start: bits from the
+// first code of axis d to the chunk's first, kMaxAxisChunks entries a meshlet
+// (ResidChunk's counterpart: a v5 meshlet has one code stream an axis).
+struct CodeChunk {
+  uint16_t pos[3];
+  uint16_t bad;   // entry 0: a position past 65,535 bits
+};
+
 // Strip tokens of a meshlet (a strip of length L has max(L, 1) triangles
 // and two more tokens).
 STRIDE_DEV uint32_t pdlt_tokens_of(const PdltEntry& e) {
@@ -114,6 +128,15 @@ STRIDE_DEV uint32_t pdlt_ref_chunks(uint32_t n_bnd) {
 // its end when it has no interior vertex.
 STRIDE_DEV uint32_t pdlt_tokens_end(const PdltEntry& e) {
   return e.n_int ? e.axis_bit[0] : e.end_bit;
+}
+
+// The words a code wave of meshlets first .. last reads: from the first
+// one's residual section to the last one's end, with the streams' read-ahead;
+// runs of more than kCodeWords are not staged.
+constexpr uint64_t kCodeWords = 4096;
+STRIDE_DEV uint64_t pdlt_code_lo(const PdltEntry& first) { return pdlt_tokens_end(first) >> 5; }
+STRIDE_DEV uint64_t pdlt_code_words(const PdltEntry& first, const PdltEntry& last) {
+  return (((uint64_t)last.end_bit - 1) >> 5) + 6 - pdlt_code_lo(first);
 }
 
 // Decode constants, widened to float64 as the reference decoder does.
@@ -200,7 +223,12 @@ STRIDE_DEV uint32_t v5_scan_unary(BitReader<Src>& r, uint64_t end_all, uint64_t 
 // ---------------------------------------------------------------------------
 template <class Src>
 STRIDE_DEV uint32_t pdlt_scan(const Src& src, uint32_t start, uint64_t end_all,
-                              uint64_t n_boundary, PdltEntry& e) {
+                              uint64_t n_boundary, PdltEntry& e, CodeChunk* chunks = nullptr) {
+  auto mark = [&](uint32_t i, int d, uint32_t bits) {
+    if (!chunks || i % kAxisChunk) return;
+    chunks[i / kAxisChunk].pos[d] = (uint16_t)bits;
+    if (bits > 0xFFFFu) chunks[0].bad = 1;
+  };
   BitReader<Src> r;
   r.init(src, start);
   e.start_bit = start;
@@ -271,6 +299,7 @@ STRIDE_DEV uint32_t pdlt_scan(const Src& src, uint32_t start, uint64_t end_all,
         const int64_t mn = (mu & 0x8000u) ? (int64_t)mu - 0x10000 : (int64_t)mu;
         const uint32_t bw = r.bits(8);
         if (bw > 32) return kV5ErrRange;
+        for (uint32_t i = 0; i < e.n_int; i += kAxisChunk) mark(i, d, bw * i);
         if (mn + (int64_t)((1ull << bw) - 1) > 0x7FFFFFFFll) {
           for (uint32_t i = 0; i < e.n_int; ++i)
             if (mn + (int64_t)r.bits((int)bw) > 0x7FFFFFFFll) return kV5ErrRange;
@@ -282,7 +311,9 @@ STRIDE_DEV uint32_t pdlt_scan(const Src& src, uint32_t start, uint64_t end_all,
       } else if (tag == 1 || tag == 2) {
         const uint32_t k = r.bits(8);
         if (k > 31) return kV5ErrRange;
+        const uint32_t first = r.pos;
         for (uint32_t i = 0; i < e.n_int; ++i) {
+          mark(i, d, r.pos - first);
           uint64_t q;
           const uint32_t err = v5_scan_unary(r, end_all, tag == 1 ? (1ull << (32 - k)) : 32ull, q);
           if (err) return err;
@@ -505,6 +536,98 @@ STRIDE_DEV void pdlt_axis(const uint32_t* __restrict__ st, int64_t rel, const Pd
       rc[v] = (T)(pred + (double)code * delta);
     }
   }
+}
+
+// A code lane: the residual codes of walk entries 32 c .. 32 c + 31 of axis
+// d to out(i, code), from a word source of the stream (pdlt_axis's codes).
+template <class Src, class Out>
+STRIDE_DEV void pdlt_code_chunk(const Src& src, const PdltEntry& e, const CodeChunk& cc, uint32_t c,
+                                int d, Out& out) {
+  const uint32_t ab = pick3(d, e.axis_bit[0], e.axis_bit[1], e.axis_bit[2]);
+  const uint32_t tag = bits_at_src(src, ab, 8);
+  const uint32_t at = pick3(d, cc.pos[0], cc.pos[1], cc.pos[2]);
+  const uint32_t left = e.n_int - (uint32_t)kAxisChunk * c;
+  const uint32_t n = left < (uint32_t)kAxisChunk ? left : (uint32_t)kAxisChunk;
+  BitStream<Src> bs;
+  if (tag == 0) {
+    const int32_t mn = (int32_t)(int16_t)(uint16_t)bits_at_src(src, (uint64_t)ab + 8, 16);
+    const uint32_t bw = bits_at_src(src, (uint64_t)ab + 24, 8);
+    bs.init(src, (uint64_t)ab + 32 + at);
+    for (uint32_t i = 0; i < n; ++i)
+      out(i, (uint32_t)((int64_t)mn + (int64_t)bs.bits(bw)));
+    return;
+  }
+  const uint32_t k = bits_at_src(src, (uint64_t)ab + 8, 8);
+  const bool eg = tag != 1;
+  const uint32_t egm = eg ? ~0u : 0u;
+  bs.init(src, (uint64_t)ab + 16 + at);
+  for (uint32_t i = 0; i < n; ++i) {
+    uint32_t u;
+    const uint32_t len = codeword_win(bs.win, egm, (int)k, u);
+    if (len) {
+      bs.drop(len);
+      out(i, (u >> 1) ^ (0u - (u & 1u)));
+    } else {
+      out(i, (uint32_t)codeword_s(bs, eg, (int)k));
+    }
+  }
+}
+
+// Eight walk entries and their codes.
+struct CodeWalk8 {
+  Walk4 a, b, p, q;
+  STRIDE_DEV void load(const Walk4* __restrict__ w, const Walk4* __restrict__ codes, uint32_t i) {
+    a = w[2 * i];
+    b = w[2 * i + 1];
+    p = codes[2 * i];
+    q = codes[2 * i + 1];
+  }
+};
+
+// pdlt_axis over decoded codes: the same arithmetic; walk and codes are read
+// from HBM eight entries ahead (whole groups of eight, one past the last).
+template <class T>
+STRIDE_DEV void pdlt_axis_codes(uint32_t n_bnd, const PdltParams& P, T* __restrict__ rc,
+                                const Walk4* __restrict__ walk, const Walk4* __restrict__ codes,
+                                uint32_t n_emit) {
+  CodeWalk8 cur, nxt;
+  cur.load(walk, codes, 0);
+  constexpr bool c32 = sizeof(T) == 4;
+  T s = 0;
+  for (uint32_t i = 0; i < n_bnd; ++i) s = s + rc[i];
+  const T fb = n_bnd ? s / (T)n_bnd : (T)0;
+  const T w0 = (T)P.w[0], w1 = (T)P.w[1], w2 = (T)P.w[2], delta = (T)P.delta;
+  auto step = [&](uint32_t ent, uint32_t code) {
+    const uint32_t v = ent & 0xFFu, a = (ent >> 8) & 0xFFu;
+    const T xa = rc[a], xb = rc[(ent >> 16) & 0xFFu], xc = rc[ent >> 24];
+    const T t0 = w0 * xa;
+    const T t1 = w1 * xb;
+    const T t2 = w2 * xc;
+    const T lin = (t0 + t1) + t2;
+    const T pred = a != v ? lin : fb;
+    rc[v] = pred + (T)(int32_t)code * delta;
+  };
+  uint32_t i = 0;
+  for (; 8 * i + 8 <= n_emit; ++i) {
+    nxt.load(walk, codes, i + 1);
+    step(cur.a.x, cur.p.x);
+    step(cur.a.y, cur.p.y);
+    step(cur.a.z, cur.p.z);
+    step(cur.a.w, cur.p.w);
+    step(cur.b.x, cur.q.x);
+    step(cur.b.y, cur.q.y);
+    step(cur.b.z, cur.q.z);
+    step(cur.b.w, cur.q.w);
+    cur = nxt;
+  }
+  const uint32_t left = n_emit - 8 * i;
+  if (left > 0) step(cur.a.x, cur.p.x);
+  if (left > 1) step(cur.a.y, cur.p.y);
+  if (left > 2) step(cur.a.z, cur.p.z);
+  if (left > 3) step(cur.a.w, cur.p.w);
+  if (left > 4) step(cur.b.x, cur.q.x);
+  if (left > 5) step(cur.b.y, cur.q.y);
+  if (left > 6) step(cur.b.z, cur.q.z);
 }
 
 // Boundary-table position as the chain starts from it.
