@@ -77,7 +77,7 @@ BENCH_CANDIDATES = ([dict(mode=2, group_size=gs, lds_bytes=lds, grid=0, use_queu
                     # waves in flight
                     + [dict(mode=4, group_size=gs, lds_bytes=16384, tok_chains=16, tok_group=tg,
                             grid=0, use_queue=0)
-                       for tg, gs in ((2, 6), (2, 8), (4, 6))]
+                       for tg, gs in ((1, 2), (2, 6), (2, 8), (4, 6), (4, 12))]
                     + [dict(mode=1, group_size=gs, lds_bytes=lds, grid=0, use_queue=0)
                        for gs in (32, 64) for lds in (16384, 40960)])
 

@@ -23,6 +23,8 @@ struct PdltSet {
   int tok_lds_budget = 16384;
   int tok_group = 4;                    // meshlets per token-pass wave
   int tok_chains = 16;                  // > 0: token chains (about this many a meshlet)
+  // until a tune names a shape, waves take meshlets by the set's size (set_layout)
+  bool auto_shape = true;
   bool chain_waves = false;             // tok_groups are chain token waves (pdlt_layout_chains)
   uint32_t n_chains = 0;                // entries at d_chains
   int chain32 = 0;                      // 1: the encoder's float32 chain

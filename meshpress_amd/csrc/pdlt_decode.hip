@@ -679,10 +679,19 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   // token lanes
   std::vector<ChainEntry> ch;
   std::vector<RefChunk> rch;
+  // Meshlets per wave of the default shape, as DecodeSet::axis_group and
+  // token_group: short waves for few meshlets.  Measured, float64 / float32,
+  // against 16 (as many as fit) and 4 throughout: 10 to 298 meshlets (2 and 1)
+  // 30 / 30 against 42 to 45 / 49 to 59 us, 913 (2 and 1) 33 / 33 against 46 /
+  // 60, 2,217 (3 and 2) 41 / 41 against 53 / 60, 8,900 (4 and 4) 62 / 59 against
+  // 65 / 75, 32,100 (6 and 4) 159 / 137 against 159 / 160.
+  const int auto_tok = H.n_m < 1024 ? 1 : H.n_m < 4096 ? 2 : 4;
+  const int auto_gs = H.n_m < 1536 ? 2 : H.n_m < 4096 ? 3 : H.n_m < 24576 ? 4 : 6;
   bool cw = false;
   int rc = STRIDE_OK;
   if (tok_chains > 0) {
-    rc = pdlt_layout_chains(tab, H.words, tok_chains, tok_group, tg, ch, rch, tlds, err);
+    rc = pdlt_layout_chains(tab, H.words, tok_chains, auto_shape ? auto_tok : tok_group, tg, ch, rch,
+                            tlds, err);
     cw = rc == STRIDE_OK;
     if (rc == STRIDE_E_UNSUPPORTED) rc = STRIDE_OK;
   }
@@ -702,7 +711,8 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   // float64 (the chain pass of the two-pass decode reads the refs from HBM;
   // its blocks keep the refs slot where pdlt_chain_block_refs says so)
   if (!rc)
-    rc = pdlt_layout(tab, gs, budget, gr, lds, err, chain32 ? 3u : 6u,
+    rc = pdlt_layout(tab, auto_shape && codes ? std::min(gs, auto_gs) : gs, budget, gr, lds, err,
+                     chain32 ? 3u : 6u,
                      two_pass == 0 || pdlt_chain_block_refs(chain32 != 0), codes);
   if (rc) return set_error(rc, err);
   if (codes && !d_codes) PDLT_HIP(hipMalloc(&d_codes, 12 * cstride()));

@@ -169,6 +169,9 @@ struct DecodeSet {
   float* d_v_own = nullptr;
   uint32_t* d_t_own = nullptr;
   DecodeConfig cfg;
+  // until set_tune names a shape, the two passes' waves take as many meshlets
+  // as suits the set's size (axis_group, token_group)
+  bool auto_shape = true;
   // group layout (mode 1)
   GroupEntry* d_groups = nullptr;
   uint32_t n_groups = 0;
@@ -350,14 +353,30 @@ struct DecodeSet {
     }
     HIP_TRY(hipMalloc(&d_v_own, 12 * std::max<uint64_t>(n_v, 1)));
     HIP_TRY(hipMalloc(&d_t_own, 12 * std::max<uint64_t>(n_t, 1)));
-    // default launch shape (the fastest measured on the 1.3M- and
-    // 7.2M-triangle meshes and the 2,048-mesh batch): 16 token chains per
-    // meshlet, 4 meshlets per token wave, axis groups of 21 meshlets
+    // default launch shape: 16 token chains per meshlet, at most 4 meshlets
+    // per token wave and axis groups of at most 21 (fewer by axis_group and
+    // token_group while no tune is set)
     cfg.tok_chains = 16;
     cfg.tok_group = 4;
     cfg.group_size = kAxisSlots;
     cfg.lds_bytes = 24576;
     return layout();
+  }
+
+  // Meshlets per wave of the default shape.  Both passes are chains of
+  // latencies: few meshlets decode fastest in short waves spread over the
+  // chip, many in full ones.  Measured, whole decodes, against 21 and 4
+  // throughout: 10 to 298 meshlets (2 and 1) 27 against 36 to 41 us, 1,287 (6
+  // and 2) 32 against 42, 4,400 (6 and 4) 42 against 48, 17,500 (12 and 4) 74
+  // against 80, 41,700 (12 and 4) 144 against 153; 32,100 is better off in
+  // groups of 21, 104 against 108.
+  int axis_group() const {
+    if (!auto_shape) return cfg.group_size;
+    return n_m < 512 ? 2 : n_m < 8192 ? 6 : 12;
+  }
+  int token_group() const {
+    if (!auto_shape || cfg.tok_chains == 0) return cfg.tok_group;
+    return n_m < 1024 ? 1 : n_m < 4096 ? 2 : 4;
   }
 
   // Partition the meshlets into groups for the current tune and run one
@@ -385,7 +404,7 @@ struct DecodeSet {
         const bool two = cfg.mode == 4;
         const bool nar = narrow_codes;
         const uint32_t gmax =
-            split ? std::min(cfg.group_size, two ? kAxisSlots : 16) : cfg.group_size;
+            split ? std::min(axis_group(), two ? kAxisSlots : 16) : cfg.group_size;
         // bytes of LDS: staged words + per-meshlet code storage ("codes"
         // counts vertices in mode 1, block words in mode 2, code words and
         // staged axis words in mode 4, whose axis pass stages nothing else)
@@ -527,7 +546,7 @@ struct DecodeSet {
       for (uint32_t gi = g_base[i]; gi < g_base[i + 1]; ++gi) {
         const GroupEntry& G = groups[gi];
         const uint64_t words = (uint64_t)G.w_lo + G.n_words - cur.w_lo;
-        if (open && G.m0 == cur.m1 && G.m1 - cur.m0 <= (uint32_t)cfg.tok_group &&
+        if (open && G.m0 == cur.m1 && G.m1 - cur.m0 <= (uint32_t)token_group() &&
             4 * words <= kTokenLds) {
           cur.m1 = G.m1;
           cur.n_words = (uint32_t)words;
@@ -621,7 +640,7 @@ struct DecodeSet {
           // look-ahead window
           const uint64_t lo = (bb + e.start_bit) >> 5;
           const uint64_t hi = ((bb + e.resid_bit + 31) >> 5) + 2;
-          if (open && j == cur.m1 && j - cur.m0 < (uint32_t)cfg.tok_group &&
+          if (open && j == cur.m1 && j - cur.m0 < (uint32_t)token_group() &&
               cur.pad[1] - cur.pad[0] + cnt <= 64 &&
               need(hi - cur.w_lo, rec_words + rw) <= kChainLds) {
             cur.m1 = j + 1;
@@ -871,9 +890,10 @@ struct DecodeSet {
       return fail(STRIDE_E_ARG, "tok_chains must be in [0, 16] (or -1 to keep)");
     const int tok_group = t->tok_group ? t->tok_group : (tok_chains > 0 ? 4 : 32);
     if (tok_group < 1 || tok_group > 64) return fail(STRIDE_E_ARG, "tok_group must be in [1, 64]");
-    const bool relayout = t->mode != cfg.mode || t->group_size != cfg.group_size ||
+    const bool relayout = auto_shape || t->mode != cfg.mode || t->group_size != cfg.group_size ||
                           t->lds_bytes != cfg.lds_bytes || tok_group != cfg.tok_group ||
                           tok_chains != cfg.tok_chains;
+    auto_shape = false;
     cfg.tok_group = tok_group;
     cfg.tok_chains = tok_chains;
     cfg.waves = t->waves;
@@ -1225,6 +1245,8 @@ int stride_decoder_set_tune(stride_decoder* h, const stride_tune* t) {
     // the refs in LDS), so it is set before the layout
     const int prev_tg = h->v5->tok_group, prev_kc = h->v5->tok_chains,
               prev_tp = h->v5->two_pass;
+    const bool prev_auto = h->v5->auto_shape;
+    h->v5->auto_shape = false;
     h->v5->tok_group = tg;
     h->v5->tok_chains = kc;
     if (t->mode) h->v5->two_pass = t->mode == 4;
@@ -1233,6 +1255,7 @@ int stride_decoder_set_tune(stride_decoder* h, const stride_tune* t) {
       h->v5->tok_group = prev_tg;
       h->v5->tok_chains = prev_kc;
       h->v5->two_pass = prev_tp;
+      h->v5->auto_shape = prev_auto;
       return rc;
     }
     return STRIDE_OK;

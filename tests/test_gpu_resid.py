@@ -103,3 +103,69 @@ def test_scan_by_waves_and_by_lanes(coracle, meshlets):
         assert np.array_equal(got[i][1].astype(np.int64), To)
         assert np.array_equal(got[i][0].view(np.uint32), Vo.view(np.uint32))
     assert all(np.array_equal(g[0].view(np.uint32), got[1][0].view(np.uint32)) for g in got[2:])
+
+
+@pytest.mark.parametrize("meshlets", [1, 511, 512, 1023, 1024])
+def test_default_shape_by_size(coracle, meshlets):
+    """The default shape's waves on both sides of their lines, against a named
+    shape (which the reported default is), single streams and batches."""
+    import torch
+    from meshpress_amd.batch import BatchDecoder
+    one = stream(*ribbon(40), 12, 3)
+    Vo, To = coracle.decode(one)
+    bd = BatchDecoder([one] * meshlets)
+    assert bd.n_meshlets == meshlets
+    shape = bd.get_tune()
+    assert (shape["group_size"], shape["tok_group"], shape["tok_chains"]) == (21, 4, 16)
+    for tune in (None, shape):
+        if tune:
+            bd.set_tune(**tune)
+        for mode in ("launch", "per_mesh", "graph"):
+            bd.d_verts.fill_(-1)
+            bd.d_tris.fill_(-1)
+            v, t = bd.decode(mode)
+            torch.cuda.synchronize()
+            v, t = v.cpu().numpy(), t.cpu().numpy()
+            for i in (0, meshlets // 2, meshlets - 1):
+                (Vi, Ti), = [bd.split(v, t)[i]]
+                assert np.array_equal(Ti.astype(np.int64), To)
+                assert np.array_equal(Vi.view(np.uint32), Vo.view(np.uint32))
+
+
+@pytest.mark.parametrize("chain", ["f64", "f32"])
+@pytest.mark.parametrize("tris", [2304, 230000, 360000])
+def test_pdlt_code_waves_match_one_kernel(tris, chain):
+    """PDLT v5 with code waves in the default shape and in named ones, against
+    the one-kernel decode of the same stream."""
+    from meshpress_amd import workloads
+    from meshpress_amd.encoder.paradelta_v5 import encode_from_prepared_v5
+    from meshpress_amd.encoder.prep import prepare
+    from meshpress_amd.utils.paradelta_v5_cuda import ParaDeltaV5GpuDecoder
+    V, T = workloads.mesh_with_tris("torus", tris, 5)
+    data = encode_from_prepared_v5(prepare(V, T, precision_error=1.0 / 4094.5, precision_mode="bbox_frac"))
+    dec = ParaDeltaV5GpuDecoder(data, chain=chain)
+    got = [dec.decode_to_host()]
+    for tune in (dict(mode=4, group_size=16, tok_group=4, tok_chains=16), dict(group_size=1, tok_group=64),
+                 dict(tok_chains=0, tok_group=64), dict(mode=3)):
+        dec.set_tune(**tune)
+        got.append(dec.decode_to_host())
+    for Vg, Tg in got[:-1]:
+        assert np.array_equal(Tg, got[-1][1])
+        assert np.array_equal(Vg.view(np.uint32), got[-1][0].view(np.uint32))
+
+
+@pytest.mark.parametrize("name", ["pdlt_hf_24_tags", "pdlt_torus_q16_tags", "pdlt_fan_parts", "pdlt_one_tri"])
+def test_pdlt_code_waves_on_every_coder(name):
+    """Golden streams of the three residual coders, and of meshlets without
+    interior or boundary vertices."""
+    import hashlib
+    from pathlib import Path
+    from meshpress_amd.utils.paradelta_v5_cuda import ParaDeltaV5GpuDecoder
+    z = np.load(Path(__file__).resolve().parent / "golden" / f"{name}.npz")
+    dec = ParaDeltaV5GpuDecoder(z["data"].tobytes())
+    for tune in (dict(), dict(mode=4, group_size=16, tok_group=64, tok_chains=1)):
+        if tune:
+            dec.set_tune(**tune)
+        V, T = dec.decode_to_host()
+        for a, key in ((V, "V_sha"), (T.astype(np.int64), "T_sha")):
+            assert hashlib.sha256(np.ascontiguousarray(a).tobytes()).hexdigest() == z[key].tobytes().hex()
