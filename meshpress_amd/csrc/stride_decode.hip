@@ -1086,13 +1086,13 @@ __global__ __launch_bounds__(64) void stride_axes_kernel(
 // The axis pass over decoded residuals (16-bit codes, irlp32_exact, every
 // code checked in range when the layout was made): three lanes per meshlet
 // run the code chains, then the wave dequantises.  A step is the walk entry's
-// addresses, three LDS reads, the prediction and a store, about 25
-// instructions; bound by the latency of that chain through LDS.  With the
-// codeword decode on the chain (stride_axes_kernel) a step is about 70 and the
-// pass took 46.7 us on 10 meshlets, 55.7 us on the 3.9M-triangle heightfield
-// and 123 us on 43,000 meshlets in 256 streams; this one 35 us and 57 us on
-// the latter two, for 9 and 18 us more in the token pass (residual waves).
-// Whole decodes: 63 -> 35, 92 -> 80 and 203 -> 153 us.
+// addresses, three LDS reads, the prediction and a store, 16 instructions,
+// bound by their number (CodeChain).  With the codeword decode on the chain
+// (stride_axes_kernel) a step is about 70: that pass took 46.7 us on 10
+// meshlets, 55.7 us on the 3.9M-triangle heightfield and 123 us on 43,000
+// meshlets in 256 streams; this one takes 12.6, 26 and 44 us, for 7 and 18 us
+// more in the token pass of the latter two (residual waves).  Whole decodes:
+// 63 -> 23, 92 -> 71 and 203 -> 137 us, by the launch shape in part.
 __global__ __launch_bounds__(64) void stride_code_axes_kernel(
     const MeshletEntry* __restrict__ tab, const MeshParams* __restrict__ meshes,
     const GroupEntry* __restrict__ groups, const uint32_t* __restrict__ walk_g,
