@@ -552,10 +552,12 @@ __global__ __launch_bounds__(64) void pdlt_chain_kernel(
 // Two-pass decode, pass 2 over decoded codes: a block holds a meshlet's three
 // reconstructions alone; the boundary ones are gathered, three lanes a
 // meshlet run the chains (walk and codes from HBM), the wave writes the
-// interior vertices.  Bound by the latency of the chain through LDS.  With
+// interior vertices.  Bound by the instructions of the chain, 12 a step
+// (ByteIndexed addresses, two groups of eight without copies).  With
 // the codeword decode on the chain and the walk, seen set and bits in LDS
 // (pdlt_chain_kernel) the pass took 46.6 us on the 498,000-triangle heightfield
-// (float64) and 49.2 us on the 199,800-triangle sphere (float32).
+// (float64) and 49.2 us on the 199,800-triangle sphere (float32), with shifts
+// and masks for addresses 21.1 and 19.4; now 18.4 and 15.2.
 template <class R>
 __global__ __launch_bounds__(64) void pdlt_code_chain_kernel(
     const PdltEntry* __restrict__ tab, const PdltGroup* __restrict__ groups,

@@ -592,33 +592,47 @@ STRIDE_DEV void pdlt_axis_codes(uint32_t n_bnd, const PdltParams& P, T* __restri
                                 uint32_t n_emit) {
   CodeWalk8 cur, nxt;
   cur.load(walk, codes, 0);
-  constexpr bool c32 = sizeof(T) == 4;
   T s = 0;
   for (uint32_t i = 0; i < n_bnd; ++i) s = s + rc[i];
   const T fb = n_bnd ? s / (T)n_bnd : (T)0;
   const T w0 = (T)P.w[0], w1 = (T)P.w[1], w2 = (T)P.w[2], delta = (T)P.delta;
+  ByteIndexed<T> at(rc);
   auto step = [&](uint32_t ent, uint32_t code) {
-    const uint32_t v = ent & 0xFFu, a = (ent >> 8) & 0xFFu;
-    const T xa = rc[a], xb = rc[(ent >> 16) & 0xFFu], xc = rc[ent >> 24];
+    const uint32_t v = at.template addr<0>(ent), a = at.template addr<1>(ent);
+    const T xa = at.load(a), xb = at.load(at.template addr<2>(ent)),
+            xc = at.load(at.template addr<3>(ent));
     const T t0 = w0 * xa;
     const T t1 = w1 * xb;
     const T t2 = w2 * xc;
-    const T lin = (t0 + t1) + t2;
+    T lin = (t0 + t1) + t2;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("" : "+v"(lin));   // a select, not a branch around the reads
+#endif
     const T pred = a != v ? lin : fb;
-    rc[v] = pred + (T)(int32_t)code * delta;
+    at.store(v, pred + (T)(int32_t)code * delta);
+  };
+  auto eight = [&](const CodeWalk8& g) {
+    step(g.a.x, g.p.x);
+    step(g.a.y, g.p.y);
+    step(g.a.z, g.p.z);
+    step(g.a.w, g.p.w);
+    step(g.b.x, g.q.x);
+    step(g.b.y, g.q.y);
+    step(g.b.z, g.q.z);
+    step(g.b.w, g.q.w);
   };
   uint32_t i = 0;
-  for (; 8 * i + 8 <= n_emit; ++i) {
+  for (; 8 * i + 16 <= n_emit; i += 2) {   // two groups a trip: no copies
     nxt.load(walk, codes, i + 1);
-    step(cur.a.x, cur.p.x);
-    step(cur.a.y, cur.p.y);
-    step(cur.a.z, cur.p.z);
-    step(cur.a.w, cur.p.w);
-    step(cur.b.x, cur.q.x);
-    step(cur.b.y, cur.q.y);
-    step(cur.b.z, cur.q.z);
-    step(cur.b.w, cur.q.w);
+    eight(cur);
+    cur.load(walk, codes, i + 2);
+    eight(nxt);
+  }
+  if (8 * i + 8 <= n_emit) {
+    nxt.load(walk, codes, i + 1);
+    eight(cur);
     cur = nxt;
+    ++i;
   }
   const uint32_t left = n_emit - 8 * i;
   if (left > 0) step(cur.a.x, cur.p.x);

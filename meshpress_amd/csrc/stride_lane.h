@@ -1344,6 +1344,34 @@ STRIDE_DEV void resid_chunk(const Src& words, uint64_t base, const MeshletEntry&
       chunk_values(rc.roots, c, e.n_local, true), TP);
 }
 
+// An array in LDS indexed by the bytes of a walk entry: byte B becomes an
+// address by one dot product of bytes, sizeof(T) * byte B + base.
+template <class T>
+struct ByteIndexed {
+#ifdef __HIP_DEVICE_COMPILE__
+  using Ptr = __attribute__((address_space(3))) T*;
+  uint32_t base = 0;
+  STRIDE_DEV ByteIndexed() {}
+  STRIDE_DEV explicit ByteIndexed(T* x) : base((uint32_t)(uintptr_t)(Ptr)x) {}
+  template <int B>
+  STRIDE_DEV uint32_t addr(uint32_t w) const {
+    return __builtin_amdgcn_udot4(w, (uint32_t)sizeof(T) << (8 * B), base, false);
+  }
+  STRIDE_DEV T load(uint32_t a) const { return *(Ptr)(uintptr_t)a; }
+  STRIDE_DEV void store(uint32_t a, T x) const { *(Ptr)(uintptr_t)a = x; }
+#else
+  T* base = nullptr;
+  STRIDE_DEV ByteIndexed() {}
+  STRIDE_DEV explicit ByteIndexed(T* x) : base(x) {}
+  template <int B>
+  STRIDE_DEV uint32_t addr(uint32_t w) const {
+    return (w >> (8 * B)) & 0xFFu;
+  }
+  STRIDE_DEV T load(uint32_t a) const { return base[a]; }
+  STRIDE_DEV void store(uint32_t a, T x) const { base[a] = x; }
+#endif
+};
+
 // One axis lane over decoded residuals: the code chain of axis d along the
 // walk, 16-bit codes, irlp32_exact.  Codes and residuals are taken modulo
 // 2^16: the caller has checked (AxisChain, CHECK) that every code of the
@@ -1363,26 +1391,7 @@ STRIDE_DEV void resid_chunk(const Src& words, uint64_t base, const MeshletEntry&
 struct CodeChain {
   int32_t n0, n1, n2, K, rnd;
   uint32_t prev = 0;
-#ifdef __HIP_DEVICE_COMPILE__
-  using Codes = __attribute__((address_space(3))) uint16_t*;
-  uint32_t base;
-  STRIDE_DEV void codes(uint16_t* c) { base = (uint32_t)(uintptr_t)(Codes)c; }
-  template <int B>
-  STRIDE_DEV uint32_t addr(uint32_t w) const {
-    return __builtin_amdgcn_udot4(w, 2u << (8 * B), base, false);
-  }
-  STRIDE_DEV uint32_t load(uint32_t a) const { return *(Codes)(uintptr_t)a; }
-  STRIDE_DEV void store(uint32_t a, uint32_t c) const { *(Codes)(uintptr_t)a = (uint16_t)c; }
-#else
-  uint16_t* base;
-  void codes(uint16_t* c) { base = c; }
-  template <int B>
-  uint32_t addr(uint32_t w) const {
-    return (w >> (8 * B)) & 0xFFu;
-  }
-  uint32_t load(uint32_t a) const { return base[a]; }
-  void store(uint32_t a, uint32_t c) const { base[a] = (uint16_t)c; }
-#endif
+  ByteIndexed<uint16_t> at;
   STRIDE_DEV void init(const MeshParams& P, int d) {
     n0 = (int32_t)(int16_t)pick3(d, (uint32_t)P.pred_n[0], (uint32_t)P.pred_n[3],
                                  (uint32_t)P.pred_n[6]);
@@ -1406,11 +1415,11 @@ struct CodeChain {
   }
   // w: walk entry, r: its residual in the low 16 bits
   STRIDE_DEV void step(uint32_t w, uint32_t r) {
-    const uint32_t v = addr<0>(w), a = addr<1>(w);
-    const uint32_t ca = load(a), cb = load(addr<2>(w)), cc = load(addr<3>(w));
+    const uint32_t v = at.addr<0>(w), a = at.addr<1>(w);
+    const uint32_t ca = at.load(a), cb = at.load(at.addr<2>(w)), cc = at.load(at.addr<3>(w));
     const uint32_t pred = (uint32_t)(mad(n2, cc, mad(n1, cb, mad(n0, ca, rnd))) >> K);
     prev = (a == v ? prev : pred) + r;
-    store(v, prev);
+    at.store(v, (uint16_t)prev);
   }
 };
 
@@ -1431,7 +1440,7 @@ struct Walk8 {
 // groups of eight, one past the last: up to entry (n / 8 + 1) * 8 + 7.
 STRIDE_DEV void code_chain(CodeChain& ax, uint32_t n, const Walk4* __restrict__ walk,
                            const uint32_t* __restrict__ resid, uint16_t* __restrict__ codes) {
-  ax.codes(codes);
+  ax.at = ByteIndexed<uint16_t>(codes);
   auto eight = [&](const Walk8& q) {
     ax.step(q.a.x, q.r[0]);
     ax.step(q.a.y, q.r[0] >> 16);
