@@ -251,25 +251,30 @@ struct MtfLite {
   uint64_t lo, hi;
   uint32_t n;
   STRIDE_DEV void clear() { lo = 0; hi = 0; n = 0; }
-  // entry j < 16.  A mask blend, not a select of the two halves: a select of
-  // two loads folds into one load through a computed address, which keeps
-  // a stepper's state out of registers.
+  // entry j < 16: two byte selects and a choice (the token lanes are bound by
+  // their instructions: 4 here against 8 with 64-bit shifts and masks)
   STRIDE_DEV uint32_t rank(uint32_t j) const {
-    const uint32_t sh = 8 * (j & 7);
-    const uint64_t m = 0ull - (uint64_t)(j >> 3);   // ones for j in [8, 16)
-    return (uint32_t)(((lo >> sh) & ~m) | ((hi >> sh) & m)) & 0xFFu;
+#ifdef __HIP_DEVICE_COMPILE__
+    const uint32_t sel = (j & 7u) | 0x0C0C0C00u;   // 0x0C: a zero byte
+    const uint32_t l = __builtin_amdgcn_perm((uint32_t)(lo >> 32), (uint32_t)lo, sel);
+    const uint32_t h = __builtin_amdgcn_perm((uint32_t)(hi >> 32), (uint32_t)hi, sel);
+    return j < 8 ? l : h;
+#else
+    return (uint32_t)((j < 8 ? lo : hi) >> (8 * (j & 7))) & 0xFFu;
+#endif
   }
+  // j <= 16: entries [0, j) one rank back, v in front; j >= 15 drops
+  // the last
   STRIDE_DEV void to_front(uint32_t j, uint32_t v) {
-    // bytes [0, j] of the low half: all ones >> (56 - 8 min(j, 7))
-    const uint32_t jl = j < 7 ? j : 7u;
-    const uint64_t ml = ~0ull >> (56u - 8u * jl);
-    // bytes [8, j] of the high half (none when j < 8)
-    const uint32_t jh = j < 8 ? 0u : (j - 8 < 7 ? j - 8 : 7u);
-    const uint64_t mh = j < 8 ? 0ull : (~0ull >> (56u - 8u * jh));
+    const uint32_t j8 = 8 * j;
+    // the bytes kept: those past j
+    const uint64_t kl = ~0xFFull << (j8 < 56 ? j8 : 56u);
+    const uint32_t jh = j8 - 64;   // wraps for j < 8
+    const uint64_t kh = j8 < 64 ? ~0ull : ~0xFFull << (jh < 56 ? jh : 56u);
     const uint64_t sl = (lo << 8) | (uint64_t)(v & 0xFFu);
     const uint64_t sh = (hi << 8) | (lo >> 56);
-    lo = (lo & ~ml) | (sl & ml);
-    hi = (hi & ~mh) | (sh & mh);
+    lo = (lo & kl) | (sl & ~kl);
+    hi = (hi & kh) | (sh & ~kh);
   }
   // 0x80 in each zero byte of x
   STRIDE_DEV static uint32_t zero_bytes(uint32_t x) {

@@ -319,15 +319,18 @@ struct LdsCursor {            // staged words in LDS
   // the next 32 bits as the two words holding them: read now, combined
   // (window()) where the bits are needed, so the reads' latency passes
   // under the work in between
+  // The words at bit pc - 1 (tokens never start a staged range: a header
+  // comes before them), so that the 32 bits end 0..31 bits before the second
+  // word's end, which one shift of the pair reaches.
   struct Raw {
-    uint32_t a, b, sh;
+    uint32_t a, b, sh;   // sh: its low five bits count
   };
   STRIDE_DEV Raw peek_raw() const {
-    const uint32_t w = pc >> 5;
-    return Raw{st[w], st[w + 1], pc & 31u};
+    const uint32_t q = pc - 1u, w = q >> 5;
+    return Raw{st[w], st[w + 1], ~q};
   }
   STRIDE_DEV static uint32_t window(const Raw& r) {
-    return (r.a << r.sh) | ((r.b >> 1) >> (31u - r.sh));
+    return (uint32_t)((((uint64_t)r.a << 32) | r.b) >> (r.sh & 31u));   // v_alignbit_b32
   }
 };
 
@@ -592,6 +595,10 @@ STRIDE_DEV void chain_starts(const Src& src, uint32_t start, const MeshletEntry&
 }
 
 // Phase 1: the lane of one chain, over a Cursor (LdsCursor in the kernel).
+// Bound by its instructions (VALU issue 88 % busy on large meshes): 63 a token,
+// of which the strip's state takes 20, the bits 12 and the FIFO 25; 74 with
+// the FIFO in 64-bit shifts, the window in four instructions and the code
+// below it in selects (46.4 -> 44.2 us for the pass on 3.9 million triangles).
 // kZeroLen: strips of length 0 occur (PDLT v5) and take three tokens.
 template <class Cursor, bool kZeroLen = false>
 struct ChainLane {
@@ -621,14 +628,11 @@ struct ChainLane {
     fifo.n = n;
     // placeholders: rank r holds n_local + r (chains after the first only;
     // the first chain starts with an empty FIFO)
-    uint64_t lo = 0, hi = 0;
-    for (uint32_t r = 0; r < 16; ++r) {
-      const uint64_t b = (uint64_t)((n_local + r) & 0xFFu);
-      if (r < 8) lo |= b << (8 * r);
-      else hi |= b << (8 * (r - 8));
-    }
-    fifo.lo = ci ? lo : 0ull;
-    fifo.hi = ci ? hi : 0ull;
+    // n_local + 15 < 256 where there is more than one chain: no byte carries
+    const uint32_t p0 = byte4(n_local & 0xFFu) + 0x03020100u;
+    const uint32_t p1 = p0 + 0x04040404u;
+    fifo.lo = ci ? ((uint64_t)p1 << 32) | p0 : 0ull;
+    fifo.hi = ci ? fifo.lo + 0x0808080808080808ull : 0ull;
     Wn = cur.peek_raw();
   }
   STRIDE_DEV bool done() const { return t >= t1; }
@@ -639,21 +643,20 @@ struct ChainLane {
     const bool start = j == lp2;
     const uint32_t L = W >> 16;
     lp2 = start ? (kZeroLen && L == 0 ? 1u : L) + 2u : lp2;
-    W = start ? (W << 16) : W;
     j = start ? 0u : j;
     const bool root = j < 3;
+    // the bits before the flag: a strip's length, then the edge bit
+    const uint32_t ls = start ? 16u : 0u, lr = root ? 0u : 1u;
+    W <<= ls;
     const uint32_t ec = root ? 0u : (W >> 31);
-    W = root ? W : (W << 1);
-    const uint32_t flag = W >> 31;
-    const uint32_t val = flag ? ((W << 1) >> (32 - ib)) : ((W >> 26) & 31u);
-    cur.advance((start ? 16u : 0u) + (root ? 1u : 2u) + (flag ? ib : 5u));
+    W <<= lr;
+    const bool hit = (int32_t)W >= 0;
+    const uint32_t val = hit ? W >> 26 : (W << 1) >> (32 - ib);
+    cur.advance(ls + lr + (hit ? 6u : ib + 1u));
     Wn = cur.peek_raw();
-    const bool hit = flag == 0;
     uint32_t jf = hit ? ((fifo.n - 1 - val) & 15u) : fifo.n;
-    // the hit's entry, read on every token and blended in: a select here
-    // compiles to a branch around the read
-    const uint32_t hm = 0u - (uint32_t)hit;
-    const uint32_t v = (fifo.rank(jf) & hm) | (val & 0xFFu & ~hm);
+    const uint32_t rk = fifo.rank(jf & 15u);
+    const uint32_t v = hit ? rk : val & 0xFFu;
     if constexpr (kFind) {
       if (raw_in_fifo && !hit) {
         const int pf = fifo.find(v);
