@@ -387,7 +387,7 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
   // the chain lane's meshlet: the count of chain-index-0 entries up to the
   // lane, less one (the wave's chains run meshlet by meshlet)
   const bool chain_lane = (uint32_t)lane < nch;
-  const uint64_t starts = __ballot(chain_lane && ((ce.state >> 24) & 15u) == 0u);
+  const uint64_t starts = __builtin_amdgcn_ballot_w64(chain_lane && ((ce.state >> 24) & 15u) == 0u);
   const uint32_t mi =
       chain_lane ? lanes_below(starts) - (((ce.state >> 24) & 15u) != 0u ? 1u : 0u) : 0u;
   const uint32_t c_roff = __shfl(roff, (int)mi, 64);
@@ -399,7 +399,7 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
   // the chunk lane's meshlet, found as the chain lane's
   const bool chunk_lane = (uint32_t)lane < nrc;
   const uint32_t rci = rk.pos >> 16;
-  const uint64_t rstarts = __ballot(chunk_lane && rci == 0u);
+  const uint64_t rstarts = __builtin_amdgcn_ballot_w64(chunk_lane && rci == 0u);
   const uint32_t ri = chunk_lane ? lanes_below(rstarts) - (rci != 0u ? 1u : 0u) : 0u;
   const uint32_t r_start = __shfl(e.start_bit, (int)ri, 64);
   const uint32_t r_nb = __shfl(e.n_bnd, (int)ri, 64);
@@ -442,8 +442,9 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
     for (uint32_t t = lane; t < nt; t += 64) {
       const uint32_t r = rj[t];
       const uint32_t v = r & 0xFFu;
-      const uint32_t ci = r >> 12;
-      const uint32_t pv = fb[16 * (cb + (ci ? ci - 1 : 0u)) + ((v - nl) & 15u)];
+      // chain c takes the FIFO of chain c - 1; the first chain has none to
+      // take (it reads the LDS words below the FIFOs and drops them)
+      const uint32_t pv = fb[(int)(16 * (cb + (r >> 12)) + ((v - nl) & 15u)) - 16];
       const uint32_t rv = v >= nl ? pv : v;   // placeholders only in chains c >= 1
       rj[t] = (uint16_t)((r & 0xFF00u) | rv);
       atomicMin(first + rv, gen | t);
@@ -470,11 +471,13 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
       const uint32_t rr = rj[act ? t : nt - 1];
       const uint32_t r = act ? rr : kRecRoot;
       const uint32_t v = r & 0xFFu;
-      const bool fresh = act && v >= nb && first[v] == (gen | t);
+      // a lane past the last token is a root without a triangle whose t no
+      // local was first seen at: its flags come out false by themselves
+      const bool fresh = first[v] == (gen | t) && v >= nb;
       const int iv1 = wave_shr1((int)v, cv1);
       const int iv2 = wave_shr1(iv1, cv2);
       const uint32_t key =
-          (act && (r & kRecEc) == 0) ? ((t << 8) | ((uint32_t)iv2 & 0xFFu)) + 1u : 0u;
+          (r & kRecEc) == 0 ? ((t << 8) | ((uint32_t)iv2 & 0xFFu)) + 1u : 0u;
       const uint32_t inc = wave_incl_max(key);
       const uint32_t s = max((uint32_t)wave_shr1((int)inc, 0), carry);
       cv1 = __builtin_amdgcn_readlane((int)v, 63);
@@ -485,8 +488,9 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
       const uint32_t p0 = (s - 1u) & 0xFFu;
       uint32_t a, b;
       const uint32_t entry = chain_entry(r, v1, v2, p0, a, b);
-      const bool emit = act && chain_emits(r);
-      const uint64_t bf = __ballot(fresh), be = __ballot(emit);
+      const bool emit = chain_emits(r);
+      const uint64_t bf = __builtin_amdgcn_ballot_w64(fresh);
+      const uint64_t be = __builtin_amdgcn_ballot_w64(emit);
       const uint32_t widx = wbase + lanes_below(bf), tidx = tbase + lanes_below(be);
       wbase += (uint32_t)__popcll(bf);
       tbase += (uint32_t)__popcll(be);
@@ -504,7 +508,7 @@ __global__ __launch_bounds__(64) void pdlt_chain_tokens_kernel(
 #pragma unroll
     for (uint32_t q = 0; q < 4; ++q) {
       const uint32_t i = 64u * q + (uint32_t)lane;
-      const uint64_t sb = __ballot(i < nb || (first[i] >> 16) == 63u - j);
+      const uint64_t sb = __builtin_amdgcn_ballot_w64(i < nb || (first[i] >> 16) == 63u - j);
       if (lane == 0) {
         so[2 * q] = (uint32_t)sb;
         so[2 * q + 1] = (uint32_t)(sb >> 32);

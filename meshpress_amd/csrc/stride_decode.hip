@@ -939,8 +939,9 @@ __global__ __launch_bounds__(64) void stride_chain_tokens_kernel(
     for (uint32_t t = lane; t < nt; t += 64) {
       const uint32_t r = rj[t];
       const uint32_t v = r & 0xFFu;
-      const uint32_t ci = r >> 12;
-      const uint32_t pv = fb[16 * (cb + (ci ? ci - 1 : 0u)) + ((v - nl) & 15u)];
+      // chain c takes the FIFO of chain c - 1; the first chain has none to
+      // take (it reads the LDS words below the FIFOs and drops them)
+      const uint32_t pv = fb[(int)(16 * (cb + (r >> 12)) + ((v - nl) & 15u)) - 16];
       const uint32_t rv = v >= nl ? pv : v;   // placeholders only in chains c >= 1
       rj[t] = (uint16_t)((r & 0xFF00u) | rv);
       atomicMin(first + rv, gen | t);
@@ -959,13 +960,15 @@ __global__ __launch_bounds__(64) void stride_chain_tokens_kernel(
       const uint32_t rr = rj[act ? t : nt - 1];
       const uint32_t r = act ? rr : kRecRoot;
       const uint32_t v = r & 0xFFu;
-      const bool fresh = act && first[v] == (gen | t);
+      // a lane past the last token is a root without a triangle whose t no
+      // local was first seen at: its flags come out false by themselves
+      const bool fresh = first[v] == (gen | t);
       // v_{t-1}, v_{t-2} by wave shifts; p0 = v_{s-2} of the last edge-bit-0
       // token s before t by a max scan over 1 + (s << 8 | v_{s-2})
       const int iv1 = wave_shr1((int)v, cv1);
       const int iv2 = wave_shr1(iv1, cv2);
       const uint32_t key =
-          (act && (r & kRecEc) == 0) ? ((t << 8) | ((uint32_t)iv2 & 0xFFu)) + 1u : 0u;
+          (r & kRecEc) == 0 ? ((t << 8) | ((uint32_t)iv2 & 0xFFu)) + 1u : 0u;
       const uint32_t inc = wave_incl_max(key);
       const uint32_t s = max((uint32_t)wave_shr1((int)inc, 0), carry);
       cv1 = __builtin_amdgcn_readlane((int)v, 63);
@@ -976,8 +979,9 @@ __global__ __launch_bounds__(64) void stride_chain_tokens_kernel(
       const uint32_t p0 = (s - 1u) & 0xFFu;
       uint32_t a, b;
       const uint32_t entry = chain_entry(r, v1, v2, p0, a, b);
-      const bool emit = act && chain_emits(r);
-      const uint64_t bf = __ballot(fresh), be = __ballot(emit);
+      const bool emit = chain_emits(r);
+      const uint64_t bf = __builtin_amdgcn_ballot_w64(fresh);
+      const uint64_t be = __builtin_amdgcn_ballot_w64(emit);
       const uint32_t widx = wbase + lanes_below(bf), tidx = tbase + lanes_below(be);
       wbase += (uint32_t)__popcll(bf);
       tbase += (uint32_t)__popcll(be);

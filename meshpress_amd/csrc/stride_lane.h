@@ -688,7 +688,7 @@ STRIDE_DEV uint32_t chain_entry(uint32_t rec, uint32_t v1, uint32_t v2, uint32_t
   return (byte4(v) & rm) | ((v | (a << 8) | (b << 16) | (c << 24)) & ~rm);
 }
 STRIDE_DEV bool chain_emits(uint32_t rec) {
-  return (rec & kRecRoot) == 0 || (rec & kRecRoot2) != 0;
+  return (rec & (kRecRoot | kRecRoot2)) != kRecRoot;   // kRecRoot2: of a root alone
 }
 
 // Walk sinks: the whole walk in one array.  WalkArray stores first
@@ -1283,29 +1283,38 @@ struct Codewords {
 template <>
 struct Codewords<LdsStaged> {
   LdsStaged src;
-  uint32_t pos;   // bits from the first staged word
+  // one bit before the position, counted from the start of LDS (of the array
+  // on the host): a codeword never starts a staged range, and the 32 bits at
+  // the position are then one funnel shift of the words at q
+  uint32_t q;
+#ifdef __HIP_DEVICE_COMPILE__
+  using Word = const __attribute__((address_space(3))) uint32_t*;
+  STRIDE_DEV uint32_t origin() const { return 8u * (uint32_t)(uintptr_t)(Word)src.s; }
+  STRIDE_DEV uint32_t word(uint32_t i) const { return ((Word)(uintptr_t)((q >> 3) & ~3u))[i]; }
+#else
+  STRIDE_DEV uint32_t origin() const { return 0; }
+  STRIDE_DEV uint32_t word(uint32_t i) const { return src.s[(q >> 5) + i]; }
+#endif
   STRIDE_DEV void init(const LdsStaged& st, uint64_t bit) {
     src = st;
-    pos = (uint32_t)(bit - 32ull * st.lo);
-  }
-  STRIDE_DEV uint64_t window() const {
-    const uint32_t w = pos >> 5;
-    return (((uint64_t)src.s[w] << 32) | src.s[w + 1]) << (pos & 31u);
+    q = origin() + (uint32_t)(bit - 32ull * st.lo) - 1u;
   }
   template <bool RICE>
   STRIDE_DEV uint32_t next(bool eg, uint32_t egm, int k) {
-    const uint64_t W = window();   // at least 33 bits, 32 are looked at
+    const uint32_t W =
+        (uint32_t)((((uint64_t)word(0) << 32) | word(1)) >> (~q & 31u));   // v_alignbit_b32
     uint32_t u;
-    const uint32_t len = RICE ? codeword_rice(W, k, u) : codeword_win(W, egm, k, u);
+    const uint32_t len = RICE ? codeword_rice((uint64_t)W << 32, k, u)
+                              : codeword_win((uint64_t)W << 32, egm, k, u);
     if (!len) {
       BitStream<LdsStaged> s;
-      s.init(src, 32ull * src.lo + pos);
+      s.init(src, 32ull * src.lo + (q + 1u - origin()));
       const uint32_t r = (uint32_t)codeword_s(s, eg, k);
       // the window ends where the word read ahead begins
-      pos = (uint32_t)(32ull * (s.next - 1 - src.lo)) - s.valid;
+      q = origin() + (uint32_t)(32ull * (s.next - 1 - src.lo)) - s.valid - 1u;
       return r;
     }
-    pos += len;
+    q += len;
     return (u >> 1) ^ (0u - (u & 1u));
   }
 };
