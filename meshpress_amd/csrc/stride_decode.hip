@@ -1096,7 +1096,7 @@ __global__ __launch_bounds__(64) void stride_axes_kernel(
 // meshlets, 55.7 us on the 3.9M-triangle heightfield and 123 us on 43,000
 // meshlets in 256 streams; this one takes 12.6, 26 and 44 us, for 7 and 18 us
 // more in the token pass of the latter two (residual waves).  Whole decodes:
-// 63 -> 23, 92 -> 71 and 203 -> 137 us, by the launch shape in part.
+// 63 -> 22, 92 -> 68 and 203 -> 132 us, by the launch shape in part.
 __global__ __launch_bounds__(64) void stride_code_axes_kernel(
     const MeshletEntry* __restrict__ tab, const MeshParams* __restrict__ meshes,
     const GroupEntry* __restrict__ groups, const uint32_t* __restrict__ walk_g,
