@@ -543,6 +543,11 @@ STRIDE_DEV uint32_t chain_end(const ChainEntry& c, uint32_t n_tok, uint32_t lm) 
   return t0 + lm < n_tok ? t0 + lm : n_tok;
 }
 
+// 1 for a strip's body token j >= 3 (it has an edge bit), 0 for its three roots;
+// j < 2^31.  Two instructions and no select, which becomes a branch where a
+// whole wave takes it together.
+STRIDE_DEV uint32_t body_token(uint32_t j) { return (2u - j) >> 31; }
+
 // The parser state at every cut of a meshlet's n_tok strip tokens, cut
 // every lm tokens (the first at bit tok_bit of src; ChainEntry.pos counts
 // from bit `base`), written to out[0 .. chain_count).  A strip of length 0
@@ -575,7 +580,7 @@ STRIDE_DEV void chain_starts_at(const Src& src, uint32_t base, uint32_t tok_bit,
       j = 0;
     }
     // edge bit (not of a root), flag, id: one window
-    const uint32_t body = (j + 253u) >> 8;   // j >= 3 (j < 259)
+    const uint32_t body = body_token(j);
     const uint32_t raw = (r.top() << body) >> 31;
     fill += raw & ((fill - 16u) >> 31);
     r.take(body + 1u + 5u + ((ib - 5u) & (0u - raw)));
@@ -1541,7 +1546,7 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
     // edge bit (not of a root), flag, FIFO index or raw id: one window.
     // Arithmetic on 0 / 1 instead of selects, which become branches where
     // the whole wave takes them together.
-    const uint32_t body = (j + 253u) >> 8;   // j >= 3 (j < 259)
+    const uint32_t body = body_token(j);
     const uint32_t T = r.top() << body;
     const uint32_t raw = T >> 31;
     const uint32_t nb = 5u + ((ib - 5u) & (0u - raw));

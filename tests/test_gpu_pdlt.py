@@ -245,3 +245,23 @@ def test_native_bench_cli_pdlt(tmp_path):
             out = json.loads(r.stdout)
             assert out["format"] == fmt and out["n_tris"] == 65536 and out["ms"] > 0
             assert out["chain"] == int(chain) and out["tune"]["group_size"] == 8
+
+
+@pytest.mark.parametrize("case", [258, 260, 400, 509, "tubes"])
+def test_strips_past_257_triangles_in_chains(case):
+    """Meshlets of up to 511 tokens in one strip are cut into token chains:
+    one strip of n triangles, and thin tubes in meshlets of 400 triangles."""
+    from meshpress_amd import workloads
+    from meshpress_amd.encoder.paradelta_v5 import encode_v5
+    from tests.test_pdlt_host import long_strip_stream, strip_lengths
+    if case == "tubes":
+        data = encode_v5(*workloads.displaced_torus(400, 3, 1.0, 0.1, 0.02, 4, 5), max_verts=256, max_tris=400)
+        assert max(L for _, L in strip_lengths(data)) > 257
+    else:
+        data = long_strip_stream(case)
+    print(f"pdlt strips past 257 triangles: {case}", flush=True)
+    for chain in ("f64", "f32"):
+        ref = PO.decode_v5(data, chain=chain)
+        assert_same(*decoder(data, chain).decode_to_host(), *ref)
+        for tune in CHAIN_LAYOUTS:
+            assert_same(*decoder(data, chain, **tune).decode_to_host(), *ref)

@@ -226,3 +226,36 @@ def test_truncated_and_bad_headers_rejected(pdlt_check, tmp_path):
     bad[0] = 0
     rc, msg, _ = run(pdlt_check, bytes(bad), tmp_path)
     assert rc == 2 and "bad magic" in msg
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 258, 259, 260, 300, 400, 509])
+def test_long_strips_cut_into_chains(pdlt_check, tmp_path, n):
+    """One strip of n triangles, n + 2 tokens: up to 511 tokens are cut into
+    chains, and the chain cuts' scan counts past the 258 tokens of the longest
+    DPR4 strip."""
+    data = long_strip_stream(n)
+    Vo, To = PO.decode_v5(data)
+    assert To.shape == (n, 3)
+    for two_pass, k0 in ((0, 16), (1, 16), (2, 1), (2, 2), (2, 5), (2, 16)):
+        rc, V, T = run(pdlt_check, data, tmp_path, two_pass=two_pass, k0=k0)
+        assert rc == 0 and same(V, T, Vo, To), (two_pass, k0)
+
+
+@pytest.mark.parametrize("mesh", ["torus", "tubes"])
+def test_long_strips_of_meshes(pdlt_check, tmp_path, mesh):
+    """Meshlets of up to 400 triangles, whose strips pass 257 triangles."""
+    from meshpress_amd import workloads as w
+    from meshpress_amd.encoder.paradelta_v5 import encode_v5
+    if mesh == "torus":
+        V, T = w.displaced_torus(60, 20, 1.0, 0.3, 0.05, 4, 5)
+    else:
+        V, T = w.displaced_torus(400, 3, 1.0, 0.1, 0.02, 4, 5)
+    data = encode_v5(V, T, max_verts=256, max_tris=400)
+    assert max(L for _, L in strip_lengths(data)) > 257
+    Vo, To = PO.decode_v5(data)
+    V32, _ = PO.decode_v5(data, chain="f32")
+    for two_pass, k0 in ((0, 16), (1, 16), (2, 2), (2, 8), (2, 16)):
+        rc, Vl, Tl = run(pdlt_check, data, tmp_path, two_pass=two_pass, k0=k0)
+        assert rc == 0 and same(Vl, Tl, Vo, To), (two_pass, k0)
+    rc, Vl, Tl = run(pdlt_check, data, tmp_path, chain32=True, two_pass=2)
+    assert rc == 0 and same(Vl, Tl, V32, To)
