@@ -193,6 +193,10 @@ int stride_decoder_header(const stride_decoder* h, float* f13, int32_t* i16);
  *   too large for a chain token wave (48 KiB of LDS with its 16-bit token
  *   records) runs the token lanes, 64 meshlets per wave, and get_tune
  *   reports tok_chains 0 and tok_group 64.
+ *   The default values of mode 4 above (all four of them) stand for the shape
+ *   by size: waves of at most so many meshlets, fewer in streams of few, as a
+ *   decoder without a tune runs.  get_tune of such a decoder reports them, and
+ *   set_tune takes them back.
  *   get_tune reports in `reserved` the meshlets decoded by mode 0. */
 typedef struct stride_tune {
   int32_t waves;

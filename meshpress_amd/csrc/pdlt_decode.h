@@ -18,13 +18,14 @@ struct PdltSet {
   std::vector<PdltGroup> tok_groups;    // token groups of the two-pass decode
   uint32_t lds_bytes = 0;               // dynamic LDS of the group launch
   uint32_t tok_lds_bytes = 0;           // dynamic LDS of the token launch
-  int group_size = 16;
-  int lds_budget = 20480;
+  // The default shape's values: they always mean the shape by size
+  // (set_layout), as in DecodeSet::by_size.
+  static constexpr int kDefGroup = 16, kDefLds = 20480, kDefTokGroup = 4, kDefChains = 16;
+  int group_size = kDefGroup;
+  int lds_budget = kDefLds;
   int tok_lds_budget = 16384;
-  int tok_group = 4;                    // meshlets per token-pass wave
-  int tok_chains = 16;                  // > 0: token chains (about this many a meshlet)
-  // until a tune names a shape, waves take meshlets by the set's size (set_layout)
-  bool auto_shape = true;
+  int tok_group = kDefTokGroup;         // meshlets per token-pass wave
+  int tok_chains = kDefChains;          // > 0: token chains (about this many a meshlet)
   bool chain_waves = false;             // tok_groups are chain token waves (pdlt_layout_chains)
   uint32_t n_chains = 0;                // entries at d_chains
   int chain32 = 0;                      // 1: the encoder's float32 chain

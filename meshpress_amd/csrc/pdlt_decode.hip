@@ -693,10 +693,12 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   // 65 / 75, 32,100 (6 and 4) 159 / 137 against 159 / 160.
   const int auto_tok = H.n_m < 1024 ? 1 : H.n_m < 4096 ? 2 : 4;
   const int auto_gs = H.n_m < 1536 ? 2 : H.n_m < 4096 ? 3 : H.n_m < 24576 ? 4 : 6;
+  const bool by_size = gs == kDefGroup && budget == kDefLds && tok_group == kDefTokGroup &&
+                       tok_chains == kDefChains;
   bool cw = false;
   int rc = STRIDE_OK;
   if (tok_chains > 0) {
-    rc = pdlt_layout_chains(tab, H.words, tok_chains, auto_shape ? auto_tok : tok_group, tg, ch, rch,
+    rc = pdlt_layout_chains(tab, H.words, tok_chains, by_size ? auto_tok : tok_group, tg, ch, rch,
                             tlds, err);
     cw = rc == STRIDE_OK;
     if (rc == STRIDE_E_UNSUPPORTED) rc = STRIDE_OK;
@@ -717,7 +719,7 @@ int PdltSet::set_layout(int gs, int budget, int tok_budget) {
   // float64 (the chain pass of the two-pass decode reads the refs from HBM;
   // its blocks keep the refs slot where pdlt_chain_block_refs says so)
   if (!rc)
-    rc = pdlt_layout(tab, auto_shape && codes ? std::min(gs, auto_gs) : gs, budget, gr, lds, err,
+    rc = pdlt_layout(tab, by_size && codes ? std::min(gs, auto_gs) : gs, budget, gr, lds, err,
                      chain32 ? 3u : 6u,
                      two_pass == 0 || pdlt_chain_block_refs(chain32 != 0), codes);
   if (rc) return set_error(rc, err);

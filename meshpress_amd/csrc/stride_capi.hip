@@ -169,9 +169,6 @@ struct DecodeSet {
   float* d_v_own = nullptr;
   uint32_t* d_t_own = nullptr;
   DecodeConfig cfg;
-  // until set_tune names a shape, the two passes' waves take as many meshlets
-  // as suits the set's size (axis_group, token_group)
-  bool auto_shape = true;
   // group layout (mode 1)
   GroupEntry* d_groups = nullptr;
   uint32_t n_groups = 0;
@@ -353,14 +350,22 @@ struct DecodeSet {
     }
     HIP_TRY(hipMalloc(&d_v_own, 12 * std::max<uint64_t>(n_v, 1)));
     HIP_TRY(hipMalloc(&d_t_own, 12 * std::max<uint64_t>(n_t, 1)));
-    // default launch shape: 16 token chains per meshlet, at most 4 meshlets
-    // per token wave and axis groups of at most 21 (fewer by axis_group and
-    // token_group while no tune is set)
-    cfg.tok_chains = 16;
-    cfg.tok_group = 4;
+    cfg.tok_chains = kDefChains;
+    cfg.tok_group = kDefTokGroup;
     cfg.group_size = kAxisSlots;
-    cfg.lds_bytes = 24576;
+    cfg.lds_bytes = kDefLds;
     return layout();
+  }
+
+  // The default launch shape: 16 token chains per meshlet, at most 4 meshlets
+  // per token wave and axis groups of at most 21, fewer by axis_group and
+  // token_group.  Those values are what get_tune reports and always mean the
+  // shape by size, however they were set: a tune that is saved and set again,
+  // or changes another field, keeps it.
+  static constexpr int kDefChains = 16, kDefTokGroup = 4, kDefLds = 24576;
+  bool by_size() const {
+    return cfg.mode == 4 && cfg.tok_chains == kDefChains && cfg.tok_group == kDefTokGroup &&
+           cfg.group_size == kAxisSlots && cfg.lds_bytes == kDefLds;
   }
 
   // Meshlets per wave of the default shape.  Both passes are chains of
@@ -371,11 +376,11 @@ struct DecodeSet {
   // against 80, 41,700 (12 and 4) 144 against 153; 32,100 is better off in
   // groups of 21, 104 against 108.
   int axis_group() const {
-    if (!auto_shape) return cfg.group_size;
+    if (!by_size()) return cfg.group_size;
     return n_m < 512 ? 2 : n_m < 8192 ? 6 : 12;
   }
   int token_group() const {
-    if (!auto_shape || cfg.tok_chains == 0) return cfg.tok_group;
+    if (!by_size()) return cfg.tok_group;
     return n_m < 1024 ? 1 : n_m < 4096 ? 2 : 4;
   }
 
@@ -890,10 +895,9 @@ struct DecodeSet {
       return fail(STRIDE_E_ARG, "tok_chains must be in [0, 16] (or -1 to keep)");
     const int tok_group = t->tok_group ? t->tok_group : (tok_chains > 0 ? 4 : 32);
     if (tok_group < 1 || tok_group > 64) return fail(STRIDE_E_ARG, "tok_group must be in [1, 64]");
-    const bool relayout = auto_shape || t->mode != cfg.mode || t->group_size != cfg.group_size ||
+    const bool relayout = t->mode != cfg.mode || t->group_size != cfg.group_size ||
                           t->lds_bytes != cfg.lds_bytes || tok_group != cfg.tok_group ||
                           tok_chains != cfg.tok_chains;
-    auto_shape = false;
     cfg.tok_group = tok_group;
     cfg.tok_chains = tok_chains;
     cfg.waves = t->waves;
@@ -1245,8 +1249,6 @@ int stride_decoder_set_tune(stride_decoder* h, const stride_tune* t) {
     // the refs in LDS), so it is set before the layout
     const int prev_tg = h->v5->tok_group, prev_kc = h->v5->tok_chains,
               prev_tp = h->v5->two_pass;
-    const bool prev_auto = h->v5->auto_shape;
-    h->v5->auto_shape = false;
     h->v5->tok_group = tg;
     h->v5->tok_chains = kc;
     if (t->mode) h->v5->two_pass = t->mode == 4;
@@ -1255,7 +1257,6 @@ int stride_decoder_set_tune(stride_decoder* h, const stride_tune* t) {
       h->v5->tok_group = prev_tg;
       h->v5->tok_chains = prev_kc;
       h->v5->two_pass = prev_tp;
-      h->v5->auto_shape = prev_auto;
       return rc;
     }
     return STRIDE_OK;
