@@ -1555,7 +1555,12 @@ int stride_encoder_write(const stride_encoder* h, const float* f13, const int32_
   H.scale = f13[3];
   H.per_coord_err = f13[4];
   for (int i = 0; i < 9; ++i) H.pred_n[i] = pred_n[i];
-  std::vector<uint8_t> bytes = write_dup(h->prep, h->res, H, tagk, h->n_threads);
+  std::vector<uint8_t> bytes;
+  try {
+    bytes = write_dup(h->prep, h->res, H, tagk, h->n_threads);
+  } catch (const std::exception& e) {
+    return fail(STRIDE_E_PREP, e.what());
+  }
   *len = bytes.size();
   if (out) {
     if (cap < bytes.size()) return fail(STRIDE_E_ARG, "output buffer too small");

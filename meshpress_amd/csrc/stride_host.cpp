@@ -12,8 +12,8 @@
 #include <atomic>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <stdexcept>
-#include <system_error>
 #include <thread>
 
 namespace stride {
@@ -1293,18 +1293,27 @@ std::vector<uint8_t> write_dup(const Prep& P, const Residuals& R, const Header& 
   for (const Plan& pl : P.plans) total_local += pl.l2g.size();
   const int nt = (int)std::max<int64_t>(1, std::min<int64_t>(n_threads, n_m / 32));
   std::vector<BitWriter> part(nt);
+  // what a range throws reaches the caller once every thread has ended
+  std::vector<std::exception_ptr> failed(nt);
   auto range = [&](int t) {
-    write_meshlets(part[t], P, R, H, tagk, n_m * t / nt, n_m * (t + 1) / nt, rel.data());
+    try {
+      write_meshlets(part[t], P, R, H, tagk, n_m * t / nt, n_m * (t + 1) / nt, rel.data());
+    } catch (...) {
+      failed[t] = std::current_exception();
+    }
   };
   std::vector<std::thread> th;
+  th.reserve(nt);
   int started = 1;
   try {
     for (; started < nt; ++started) th.emplace_back(range, started);
-  } catch (const std::system_error&) {   // no more threads: the rest runs here
+  } catch (const std::exception&) {   // no more threads, or no memory for one: the rest runs here
   }
   range(0);
   for (int t = started; t < nt; ++t) range(t);
   for (auto& x : th) x.join();
+  for (const std::exception_ptr& e : failed)
+    if (e) std::rethrow_exception(e);
   for (int t = 1; t < nt; ++t) {
     const uint64_t at = part[0].bit_pos(), n = part[t].bit_pos();
     for (int64_t m = n_m * t / nt; m < n_m * (t + 1) / nt; ++m) rel[m] += at;
