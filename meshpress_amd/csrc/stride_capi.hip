@@ -19,6 +19,7 @@
 #include "stride_err.h"
 #include "stride_host.h"
 #include "stride_lane.h"
+#include "stride_pool.h"
 
 using namespace stride;
 
@@ -149,6 +150,26 @@ int scratch_ptr(int device, uint32_t** out) {
   return STRIDE_OK;
 }
 
+// A stream to capture a graph on; nothing ever runs there.  Making one costs a
+// call 50 to 400 us (by the state of the process), as much as the rest of the
+// first graph decode of 256 streams, so a few stay idle between captures, until
+// the process ends.
+IdlePool<hipStream_t, 4> g_capture_streams;
+
+struct CaptureStream {
+  hipStream_t s = nullptr;
+  int device = -1;
+  bool whole = false;   // the capture ended well: the stream may be taken again
+  hipError_t open() {
+    const hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess || g_capture_streams.take(device, s)) return e;
+    return hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  }
+  ~CaptureStream() {
+    if (s && !(whole && g_capture_streams.put(device, s))) (void)hipStreamDestroy(s);
+  }
+};
+
 }  // namespace
 
 // One device-resident set of DPR4 streams with its side table.
@@ -192,11 +213,9 @@ struct DecodeSet {
   bool narrow_codes = true;               // narrow(), fixed by layout()
   // captured graphs keyed by (verts, tris, tune)
   std::map<std::tuple<void*, void*, int, int, int, int, int, int, int>, hipGraphExec_t> graphs;
-  hipStream_t cap_stream = nullptr;
 
   ~DecodeSet() {
     drop_graphs();
-    if (cap_stream) (void)hipStreamDestroy(cap_stream);
     (void)hipFree(d_buf);
     (void)hipFree(d_tab);
     (void)hipFree(d_mesh);
@@ -855,11 +874,13 @@ struct DecodeSet {
                                (cfg.lds_bytes * 128 + cfg.tok_group) * 32 + cfg.tok_chains);
     auto it = graphs.find(key);
     if (it == graphs.end()) {
-      if (!cap_stream) HIP_TRY(hipStreamCreateWithFlags(&cap_stream, hipStreamNonBlocking));
+      CaptureStream cap;
+      HIP_TRY(cap.open());
       hipGraph_t g = nullptr;
-      HIP_TRY(hipStreamBeginCapture(cap_stream, hipStreamCaptureModeThreadLocal));
-      int rc = enqueue(V, T, cap_stream, 0, (int)mp.size());
-      hipError_t ec = hipStreamEndCapture(cap_stream, &g);
+      HIP_TRY(hipStreamBeginCapture(cap.s, hipStreamCaptureModeThreadLocal));
+      int rc = enqueue(V, T, cap.s, 0, (int)mp.size());
+      hipError_t ec = hipStreamEndCapture(cap.s, &g);
+      cap.whole = ec == hipSuccess;
       if (rc) {
         if (g) (void)hipGraphDestroy(g);
         return rc;
