@@ -194,6 +194,8 @@ struct DecodeSet {
   GroupEntry* d_groups = nullptr;
   uint32_t n_groups = 0;
   std::vector<uint32_t> g_base;           // first group of each mesh, n_meshes + 1
+  GroupEntry* d_named = nullptr;          // groups of the no-alloc decode (named_layout)
+  uint32_t n_named = 0, named_lds = 0;
   uint32_t* d_legacy = nullptr;           // meshlets decoded by the wave-per-meshlet kernel
   // mode 4: token groups (up to 64 meshlets, unions of consecutive split
   // groups) and the walks, one word per local vertex
@@ -223,6 +225,7 @@ struct DecodeSet {
     (void)hipFree(d_v_own);
     (void)hipFree(d_t_own);
     (void)hipFree(d_groups);
+    (void)hipFree(d_named);
     (void)hipFree(d_legacy);
     (void)hipFree(d_tgroups);
     (void)hipFree(d_walk);
@@ -391,16 +394,97 @@ struct DecodeSet {
   // latencies: few meshlets decode fastest in short waves spread over the
   // chip, many in full ones.  Measured, whole decodes, against 21 and 4
   // throughout: 10 to 298 meshlets (2 and 1) 27 against 36 to 41 us, 1,287 (6
-  // and 2) 32 against 42, 4,400 (6 and 4) 42 against 48, 17,500 (12 and 4) 74
-  // against 80, 41,700 (12 and 4) 144 against 153; 32,100 is better off in
-  // groups of 21, 104 against 108.
+  // and 2) 32 against 42, 4,400 (6 and 4) 42 against 48, 17,600 (12 and 4) 65
+  // against 71, 42,600 117 against 119, 53,100 146 against 153, 41,700 in 256
+  // streams 180 against 194; at 32,000 in one stream 99 against 97.
+  // Where the axis lanes decode the codewords (use_resid() false) the short
+  // waves pay as well, 11 meshlets of 18-bit codes 69 against 94 us, 1,287 71
+  // against 82, 4,300 73 against 79, but groups of 12 do not: 17,500 144
+  // against 144, of wide weights 364 against 361, 41,700 in 256 streams 343
+  // against 341; the no-alloc decode that falls back to them 148 against 118 on
+  // 32,000 meshlets (named_layout).
   int axis_group() const {
     if (!by_size()) return cfg.group_size;
-    return n_m < 512 ? 2 : n_m < 8192 ? 6 : 12;
+    return n_m < 512 ? 2 : n_m < 8192 ? 6 : use_resid() ? 12 : cfg.group_size;
   }
   int token_group() const {
     if (!by_size()) return cfg.tok_group;
     return n_m < 1024 ? 1 : n_m < 4096 ? 2 : 4;
+  }
+
+  // The groups of at most `group` meshlets that the current tune allows, one
+  // mesh after another (base: the first of each).  Meshlets too large for any
+  // group join `legacy`, those in it are left out.  lds: the largest group's
+  // LDS bytes, code_only: those of its code arrays alone (mode 4).
+  std::vector<GroupEntry> make_groups(int group, std::vector<uint8_t>& legacy,
+                                      std::vector<uint32_t>& base, uint32_t& lds,
+                                      uint32_t& code_only) const {
+    const int n_meshes = (int)mp.size();
+    std::vector<GroupEntry> groups;
+    const uint64_t budget = (uint64_t)cfg.lds_bytes;
+    const bool split = cfg.mode != 1;
+    const bool two = cfg.mode == 4;
+    const bool nar = narrow_codes;
+    const uint32_t gmax = split ? std::min(group, two ? kAxisSlots : 16) : group;
+    // bytes of LDS: staged words + per-meshlet code storage ("codes"
+    // counts vertices in mode 1, block words in mode 2, code words and
+    // staged axis words in mode 4, whose axis pass stages nothing else)
+    auto need = [split, two](uint64_t words, uint64_t cu) {
+      return two ? 4 * cu
+                 : (split ? 4 * ((words + 3) & ~3ull) + 4 * cu : 8 * ((words + 1) / 2) + 8 * cu);
+    };
+    lds = 0;
+    code_only = 0;
+    for (int i = 0; i < n_meshes; ++i) {
+      base[i] = (uint32_t)groups.size();
+      const uint64_t bb = mp[i].blob_byte * 8ull;
+      GroupEntry cur{};
+      uint64_t codes = 0;
+      uint32_t code_words = 0;   // mode 4: the code arrays alone
+      bool open = false;
+      auto close = [&]() {
+        if (open) {
+          code_only = std::max(code_only, 4 * code_words);
+          // mode 1: packed codes after the words, in 8-byte units;
+          // mode 2: walk/codes blocks after the words, in 4-byte units
+          cur.codes_off = split ? ((cur.n_words + 3) & ~3u) : (cur.n_words + 1) / 2;
+          groups.push_back(cur);
+          lds = std::max<uint32_t>(lds, (uint32_t)need(cur.n_words, codes));
+        }
+        open = false;
+      };
+      for (uint32_t j = m_base[i]; j < m_base[i + 1]; ++j) {
+        if (legacy[j]) { close(); continue; }
+        const MeshletEntry& e = tab[j];
+        const uint64_t lo = (bb + e.start_bit) >> 5;
+        const uint64_t hi = ((bb + e.end_bit + 31) >> 5) + 2;
+        const uint64_t unit = two ? split_code_words(e.n_local, nar) + axis_stage_words(bb, e)
+                                  : (split ? split_block_words(e.n_local, nar) : e.n_local);
+        if (open && (j - cur.m0 < gmax) && need(hi - cur.w_lo, codes + unit) <= budget) {
+          cur.m1 = j + 1;
+          cur.n_words = (uint32_t)(hi - cur.w_lo);
+          codes += unit;
+          code_words += split_code_words(e.n_local, nar);
+          continue;
+        }
+        close();
+        if (need(hi - lo, unit) > budget) {   // too large for any group
+          legacy[j] = 1;
+          continue;
+        }
+        cur = GroupEntry{};
+        cur.m0 = j;
+        cur.m1 = j + 1;
+        cur.w_lo = (uint32_t)lo;
+        cur.n_words = (uint32_t)(hi - lo);
+        codes = unit;
+        code_words = split_code_words(e.n_local, nar);
+        open = true;
+      }
+      close();
+    }
+    base[n_meshes] = (uint32_t)groups.size();
+    return groups;
   }
 
   // Partition the meshlets into groups for the current tune and run one
@@ -414,80 +498,19 @@ struct DecodeSet {
     drop_graphs();
     (void)hipFree(d_groups);
     (void)hipFree(d_legacy);
+    (void)hipFree(d_named);
     d_groups = nullptr;
     d_legacy = nullptr;
+    d_named = nullptr;
+    n_named = 0;
     const int n_meshes = (int)mp.size();
     std::vector<uint8_t> legacy(n_m, cfg.mode == 0 ? 1 : 0);
     std::vector<GroupEntry> groups;
     for (int pass = 0; pass < 2; ++pass) {
       groups.clear();
       g_base.assign(n_meshes + 1, 0);
-      if (cfg.mode == 1 || cfg.mode == 2 || cfg.mode == 4) {
-        const uint64_t budget = (uint64_t)cfg.lds_bytes;
-        const bool split = cfg.mode != 1;
-        const bool two = cfg.mode == 4;
-        const bool nar = narrow_codes;
-        const uint32_t gmax =
-            split ? std::min(axis_group(), two ? kAxisSlots : 16) : cfg.group_size;
-        // bytes of LDS: staged words + per-meshlet code storage ("codes"
-        // counts vertices in mode 1, block words in mode 2, code words and
-        // staged axis words in mode 4, whose axis pass stages nothing else)
-        auto need = [split, two](uint64_t words, uint64_t cu) {
-          return two ? 4 * cu
-                     : (split ? 4 * ((words + 3) & ~3ull) + 4 * cu : 8 * ((words + 1) / 2) + 8 * cu);
-        };
-        group_lds = 0;
-        code_lds = 0;
-        for (int i = 0; i < n_meshes; ++i) {
-          g_base[i] = (uint32_t)groups.size();
-          const uint64_t bb = mp[i].blob_byte * 8ull;
-          GroupEntry cur{};
-          uint64_t codes = 0;
-          uint32_t code_words = 0;   // mode 4: the code arrays alone
-          bool open = false;
-          auto close = [&]() {
-            if (open) {
-              code_lds = std::max(code_lds, 4 * code_words);
-              // mode 1: packed codes after the words, in 8-byte units;
-              // mode 2: walk/codes blocks after the words, in 4-byte units
-              cur.codes_off = split ? ((cur.n_words + 3) & ~3u) : (cur.n_words + 1) / 2;
-              groups.push_back(cur);
-              group_lds = std::max<uint32_t>(group_lds, (uint32_t)need(cur.n_words, codes));
-            }
-            open = false;
-          };
-          for (uint32_t j = m_base[i]; j < m_base[i + 1]; ++j) {
-            if (legacy[j]) { close(); continue; }
-            const MeshletEntry& e = tab[j];
-            const uint64_t lo = (bb + e.start_bit) >> 5;
-            const uint64_t hi = ((bb + e.end_bit + 31) >> 5) + 2;
-            const uint64_t unit = two ? split_code_words(e.n_local, nar) + axis_stage_words(bb, e)
-                                      : (split ? split_block_words(e.n_local, nar) : e.n_local);
-            if (open && (j - cur.m0 < gmax) && need(hi - cur.w_lo, codes + unit) <= budget) {
-              cur.m1 = j + 1;
-              cur.n_words = (uint32_t)(hi - cur.w_lo);
-              codes += unit;
-              code_words += split_code_words(e.n_local, nar);
-              continue;
-            }
-            close();
-            if (need(hi - lo, unit) > budget) {   // too large for any group
-              legacy[j] = 1;
-              continue;
-            }
-            cur = GroupEntry{};
-            cur.m0 = j;
-            cur.m1 = j + 1;
-            cur.w_lo = (uint32_t)lo;
-            cur.n_words = (uint32_t)(hi - lo);
-            codes = unit;
-            code_words = split_code_words(e.n_local, nar);
-            open = true;
-          }
-          close();
-        }
-        g_base[n_meshes] = (uint32_t)groups.size();
-      }
+      if (cfg.mode == 1 || cfg.mode == 2 || cfg.mode == 4)
+        groups = make_groups(axis_group(), legacy, g_base, group_lds, code_lds);
       n_groups = (uint32_t)groups.size();
       if (n_groups) {
         HIP_TRY(hipMalloc(&d_groups, sizeof(GroupEntry) * n_groups));
@@ -551,7 +574,26 @@ struct DecodeSet {
       if (flag)
         return fail(STRIDE_E_UNSUPPORTED, "decoded codes exceed 32 bits (unsupported by the GPU decoder)");
     }
+    if (int rc = named_layout(legacy)) return rc;
     ready = true;
+    return STRIDE_OK;
+  }
+
+  // A no-alloc decode whose walk fits the static scratch and whose residuals
+  // do not decodes the codewords in its axis lanes.  Streams as large as that
+  // are in the default shape's groups of 12, which suit the decoded residuals
+  // alone (axis_group): a second table holds their groups of cfg.group_size.
+  int named_layout(std::vector<uint8_t>& legacy) {
+    if (mp.size() != 1 || !by_size() || !use_resid() || axis_group() == cfg.group_size ||
+        scratch_words() > kScratchWords || resid_scratch_words() <= kScratchWords)
+      return STRIDE_OK;
+    std::vector<uint32_t> base(2, 0);
+    uint32_t code_only = 0;
+    const std::vector<GroupEntry> g = make_groups(cfg.group_size, legacy, base, named_lds, code_only);
+    if (g.empty()) return STRIDE_OK;
+    HIP_TRY(hipMalloc(&d_named, sizeof(GroupEntry) * g.size()));
+    HIP_TRY(hipMemcpy(d_named, g.data(), sizeof(GroupEntry) * g.size(), hipMemcpyHostToDevice));
+    n_named = (uint32_t)g.size();
     return STRIDE_OK;
   }
 
@@ -752,6 +794,11 @@ struct DecodeSet {
     g.rcap = rcap;
     g.code_lds_bytes = code_lds;
     if (two) g.grid = 0;
+    if (n_named && !S.resid) {   // a no-alloc decode, always of the whole stream
+      g.groups = d_named;
+      g.n_groups = n_named;
+      g.lds_bytes = named_lds;
+    }
     return g;
   }
 
