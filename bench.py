@@ -27,7 +27,9 @@ Prints one JSON line with the headline throughput in Gtris/s, the decode's
 HBM roofline figures (with the VALU issue bound of the committed counter
 profile: roofline.issue_model), a CPU baseline (the C oracle on one thread,
 and under cpu_baseline.all_threads on the host's thread share, both timed on
-this host) and the other workloads under "details".
+this host) and the other workloads under "details".  The line is kept short
+enough for what reads it (result_line); the launch-shape sweeps and the
+learned comparison's rows go to stderr.
 """
 from __future__ import annotations
 
@@ -50,6 +52,25 @@ HBM_PEAK_GBS = 8000.0
 
 def log(*a):
     print("[bench]", *a, file=sys.stderr, flush=True)
+
+
+def result_line(out) -> str:
+    """The JSON line: floats to six digits, the launch-shape sweeps and the
+    learned comparison's rows, 50 of its 55 KB, on stderr instead.  A reader
+    that keeps the last 8,000 characters of the output then has it whole."""
+    def lean(x, path=""):
+        if isinstance(x, dict):
+            r = {}
+            for k, v in x.items():
+                if k == "tune_sweep_ms":
+                    log(f"{path}{k}: {json.dumps(v)}")
+                elif not (k == "per_mesh" and isinstance(v, list)):   # rows: logged one by one
+                    r[k] = lean(v, f"{path}{k}.")
+            return r
+        if isinstance(x, (list, tuple)):
+            return [lean(v, path) for v in x]
+        return float(f"{x:.6g}") if isinstance(x, float) else x
+    return json.dumps(lean(out))
 
 
 def bbox_error(bits: int) -> float:
@@ -547,7 +568,7 @@ def main():
                     tune=json.loads(a.tune) if a.tune else not a.no_autotune,
                     modes=tuple(a.batch_modes.split(",")), cache=a.batch_cache)
         mode = "graph" if "graph" in r else tuple(k for k in ("launch", "per_mesh") if k in r)[0]
-        print(json.dumps({
+        print(result_line({
             "metric": METRIC, "value": r[mode]["gtris_s"], "unit": "Gtris/s", "n_gpus": 1,
             "steps": a.steps, "warmup": a.warmup, "ms_per_step": r[mode]["ms_wall"],
             "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
@@ -630,7 +651,7 @@ def main():
         "cpu_baseline": cpu,
         "details": details,
     }
-    print(json.dumps(out), flush=True)
+    print(result_line(out), flush=True)
 
 
 if __name__ == "__main__":
