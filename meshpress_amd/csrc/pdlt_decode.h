@@ -45,8 +45,10 @@ struct PdltSet {
   int32_t* d_codes = nullptr;
   bool code_waves = false;
   uint32_t ccap = 0;
+  // (the last slot starts at most 3 words past its entries before it and 4 a
+  // meshlet, and is read up to its entry n_int + 7)
   uint64_t cstride() const { return ((uint64_t)(H.n_v - H.n_b) + 4ull * H.n_m + 16 + 3) & ~3ull; }
-  uint32_t* d_walk = nullptr;           // two-pass walks (n_v - n_b words)
+  uint32_t* d_walk = nullptr;           // two-pass walks (cstride words)
   uint32_t* d_seen = nullptr;           // two-pass seen sets + walk lengths (kSeenWords per meshlet)
   uint32_t* d_refs = nullptr;           // two-pass boundary refs (n_refs words)
   double* d_bnd = nullptr;              // boundary table, normalised f64 (n_b x 3)

@@ -585,7 +585,7 @@ struct CodeWalk8 {
 };
 
 // pdlt_axis over decoded codes: the same arithmetic; walk and codes are read
-// from HBM eight entries ahead (whole groups of eight, one past the last).
+// from HBM eight entries ahead (whole groups of eight, up to entry n_emit + 7).
 template <class T>
 STRIDE_DEV void pdlt_axis_codes(uint32_t n_bnd, const PdltParams& P, T* __restrict__ rc,
                                 const Walk4* __restrict__ walk, const Walk4* __restrict__ codes,

@@ -648,13 +648,14 @@ struct DecodeSet {
       HIP_TRY(hipMalloc(&d_tgroups, sizeof(GroupEntry) * n_tgroups));
       HIP_TRY(hipMemcpy(d_tgroups, tg.data(), sizeof(GroupEntry) * n_tgroups, hipMemcpyHostToDevice));
     }
-    // walks at 16-byte aligned slots (walk_slot): n_v + 4 words per meshlet,
-    // + 8 for the 4-entry reads past the last one
     if (!d_walk) HIP_TRY(hipMalloc(&d_walk, 4 * walk_words()));
     if (use_resid() && !d_resid) HIP_TRY(hipMalloc(&d_resid, 6 * rstride()));
     return STRIDE_OK;
   }
 
+  // Walks at 16-byte aligned slots (walk_slot).  The last one starts at most 3
+  // words past its vertices before it and 4 a meshlet, n_v - n + 3 + 4 (n_m - 1),
+  // and is read up to its entry n + 7 (code_chain): word n_v + 4 n_m + 6.
   uint64_t walk_words() const { return n_v + 4ull * n_m + 8; }
   // the residual scratch holds an entry per walk word and axis
   uint64_t rstride() const { return (walk_words() + 3) & ~3ull; }

@@ -1092,8 +1092,8 @@ __device__ __forceinline__ void copy_strided(uint32_t* __restrict__ dst,
 
 // Walk slot of global meshlet m in the two-pass walk buffer: its first
 // vertex rounded up to 4 words, + 4 words per preceding meshlet, so every
-// slot is 16-byte aligned and a 4-entry read past a slot's end stays inside
-// the next slot or the 8 words after the last.
+// slot is 16-byte aligned and holds its entries rounded up to four; reads in
+// whole groups of eight end inside the buffer (DecodeSet::walk_words).
 STRIDE_DEV uint64_t walk_slot(const MeshParams& P, const MeshletEntry& e, uint32_t m) {
   return ((P.v_base + e.v_off + 3) & ~3ull) + 4ull * m;
 }
@@ -1454,7 +1454,8 @@ struct Walk8 {
 
 // The chain of a meshlet of n entries: walk slot and residuals in HBM, read
 // eight entries (about a memory round trip of chain steps) ahead.  Reads whole
-// groups of eight, one past the last: up to entry (n / 8 + 1) * 8 + 7.
+// groups of eight, 0 to n / 8: up to entry (n / 8) * 8 + 7, n + 7 at most, also
+// for n = 0.
 STRIDE_DEV void code_chain(CodeChain& ax, uint32_t n, const Walk4* __restrict__ walk,
                            const uint32_t* __restrict__ resid, uint16_t* __restrict__ codes) {
   ax.at = ByteIndexed<uint16_t>(codes);

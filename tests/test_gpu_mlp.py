@@ -251,3 +251,22 @@ def test_fused_passes_at_tile_edges(n):
                                      _lib.stream_ptr()))
     assert torch.equal(r2, dh2) and torch.equal(r1, dh1)
     assert np.all(np.abs(host(net.g) - want) <= n * 2.0 ** -23 * size)
+
+
+@pytest.mark.parametrize("n", [4097, 16384, 16401])
+def test_sliced_gradients_within_the_bound_of_their_slices(n):
+    """With a workspace a weight gradient is a float32 sum over a slice of at
+    most 64 ceil(n / 4096) rows, then over at most 64 slices: its error is that
+    of so many additions, not of n."""
+    torch = _t()
+    net, p, x, labels = _net(n, n)
+    dx = net.features_to_device(x)
+    h1, h2, z = net.forward(dx)
+    dz, _ = net.xent(z, torch.from_numpy(labels).to("cuda"), 1.0 / n)
+    dh2, dh1 = net.backward(dx, h1, h2, dz)
+    pairs = [(host(a), host(g)) for a, g in ((dx, dh1), (h1, dh2), (h2, dz))]
+    want = np.concatenate([(a.T @ g).ravel() for a, g in pairs] + [g.sum(0) for _, g in pairs])
+    size = np.concatenate([(np.abs(a).T @ np.abs(g)).ravel() for a, g in pairs]
+                          + [np.abs(g).sum(0) for _, g in pairs])
+    additions = 64 * -(-n // 4096) + 64
+    assert np.all(np.abs(host(net.g) - want) <= additions * 2.0 ** -23 * size)
