@@ -36,14 +36,18 @@ __device__ __forceinline__ uint32_t zz32(int32_t r) {
 __device__ __forceinline__ uint64_t zz64(int64_t r) {
   return r < 0 ? ((uint64_t)(-r) << 1) - 1u : ((uint64_t)r << 1);
 }
-// floor(log2(x)) for x >= 1
-__device__ __forceinline__ uint32_t ilog2_64(uint64_t x) { return 63u - (uint32_t)__builtin_clzll(x); }
-
+// The 20 sums in 64 bits: u >> k for Rice(k); for Exp-Golomb(k) the leading
+// zeros of u + 2^k, since floor(log2((u >> k) + 1)) = 63 - k - clz(u + 2^k)
+// (coder_sum).  u + 2^7 has to fit 64 bits.
 __device__ __forceinline__ void accumulate(uint64_t u, uint64_t (&acc)[kCoders]) {
 #pragma unroll
   for (int k = 0; k < kRiceK; ++k) acc[k] += u >> k;
 #pragma unroll
-  for (int k = 0; k < kEgK; ++k) acc[kRiceK + k] += 2u * ilog2_64((u >> k) + 1);
+  for (int k = 0; k < kEgK; ++k) acc[kRiceK + k] += (uint32_t)__builtin_clzll(u + (1ull << k));
+}
+// coder j's sum of body bits without its 1 + k a value, from accumulate's sum over n values
+__device__ __forceinline__ uint64_t coder_sum(int j, uint64_t acc, uint64_t n) {
+  return j < kRiceK ? acc : 2ull * (n * (uint64_t)(63 - (j - kRiceK)) - acc);
 }
 
 // Sum over the lanes of a group of `G` lanes that share lane % STEP (powers
@@ -154,7 +158,7 @@ __global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restr
     for (int j = 0; j < kCoders; ++j) acc[j] = 0;
     for (int64_t i = b + lane; i < e; i += G) accumulate(zz32(vals[i]), acc);
 #pragma unroll
-    for (int j = 0; j < kCoders; ++j) tot[j] = body_bits(j, group_sum<1, G>(acc[j]), n);
+    for (int j = 0; j < kCoders; ++j) tot[j] = body_bits(j, coder_sum(j, group_sum<1, G>(acc[j]), n), n);
   }
   if (lane == 0 && s < n_streams) {
     if (costs) {
@@ -189,7 +193,7 @@ __global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restr
 constexpr int kIrlpWaves = 4;
 
 template <int CB, int SL, int MB>
-__global__ __launch_bounds__(64 * kIrlpWaves) void irlp_cost_kernel(
+__global__ __launch_bounds__(64 * kIrlpWaves, 4) void irlp_cost_kernel(
     const int32_t* __restrict__ A, const int32_t* __restrict__ B, const int32_t* __restrict__ C,
     const int32_t* __restrict__ Vv, const int64_t* __restrict__ off, int64_t n_m,
     const int32_t* __restrict__ cand, int S, int K, unsigned long long* __restrict__ cost,
@@ -233,7 +237,7 @@ __global__ __launch_bounds__(64 * kIrlpWaves) void irlp_cost_kernel(
     const bool small = top < (1u << 23) && weight < (1u << 23) && peak < 0x40000000ull &&
                        fits_costs32(n, 2 * (top + (peak >> K) + 1));
     uint64_t best = ~0ull;
-    if (__all(small)) {
+    if (__builtin_expect(__all(small), 1)) {
       Costs32 acc;
       acc.clear();
       const int32_t h = (int32_t)half;
@@ -282,22 +286,43 @@ __global__ __launch_bounds__(64 * kIrlpWaves) void irlp_cost_kernel(
       }
       acc.template totals<CB, G>(n, [&](int, uint64_t t) { best = t < best ? t : best; });
     } else {
-      // four coders a pass over the samples: few registers, for a path that
-      // codes past 23 bits take
+      // Codes past 23 bits.  Many candidates: every coder in one pass over the
+      // samples (60 on 4,000 meshlets 126 us, 33 on 20,000 507; five passes of
+      // four coders 402 and 1,690).  Few: four coders a pass, whose registers
+      // leave the path above its waves (1 on 20,000 meshlets 64 us).
+      constexpr int kAt = CB >= 16 ? kCoders : 4;
 #pragma unroll 1
-      for (int j0 = 0; j0 < kCoders; j0 += 4) {
-        uint64_t acc[4] = {0, 0, 0, 0};
-        for (uint64_t i = slice; i < n; i += SL) {
-          const int64_t s = (int64_t)n0 * a0[i] + (int64_t)n1 * b0[i] + (int64_t)n2 * c0[i];
-          const int64_t pred = K ? ((s + half) >> K) : s;
-          const uint64_t u = zz64((int64_t)v0[i] - pred);
+      for (int j0 = 0; j0 < kCoders; j0 += kAt) {
+        uint64_t acc[kAt];
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            acc[q] += j0 < kRiceK ? u >> (j0 + q) : 2u * ilog2_64((u >> (j0 + q - kRiceK)) + 1);
+        for (int q = 0; q < kAt; ++q) acc[q] = 0;
+        auto value = [&](int32_t x, int32_t y, int32_t z, int32_t v) {
+          const int64_t s = (int64_t)n0 * x + (int64_t)n1 * y + (int64_t)n2 * z;
+          return zz64((int64_t)v - (K ? ((s + half) >> K) : s));
+        };
+        if constexpr (kAt == kCoders) {
+          uint64_t i = slice;
+          if constexpr (SL == 1)   // two samples' scalar loads a trip
+            for (; i + 1 < n; i += 2) {
+              const int32_t x0 = a0[i], y0 = b0[i], z0 = c0[i], w0 = v0[i];
+              const int32_t x1 = a0[i + 1], y1 = b0[i + 1], z1 = c0[i + 1], w1 = v0[i + 1];
+              accumulate(value(x0, y0, z0, w0), acc);
+              accumulate(value(x1, y1, z1, w1), acc);
+            }
+          for (; i < n; i += SL) accumulate(value(a0[i], b0[i], c0[i], v0[i]), acc);
+        } else {
+          for (uint64_t i = slice; i < n; i += SL) {
+            const uint64_t u = value(a0[i], b0[i], c0[i], v0[i]);
+#pragma unroll
+            for (int q = 0; q < kAt; ++q)
+              acc[q] += j0 < kRiceK ? u >> (j0 + q)
+                                     : (uint32_t)__builtin_clzll(u + (1ull << (j0 + q - kRiceK)));
+          }
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint64_t t = body_bits(j0 + q, group_sum<CB, G>(acc[q]), n);
+        for (int q = 0; q < kAt; ++q) {
+          const uint64_t t =
+              body_bits(j0 + q, coder_sum(j0 + q, group_sum<CB, G>(acc[q]), n), n);
           best = t < best ? t : best;
         }
       }
