@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restr
 constexpr int kIrlpWaves = 4;
 
 template <int CB, int SL, int MB>
-__global__ __launch_bounds__(64 * kIrlpWaves, 4) void irlp_cost_kernel(
+__global__ __launch_bounds__(64 * kIrlpWaves) void irlp_cost_kernel(
     const int32_t* __restrict__ A, const int32_t* __restrict__ B, const int32_t* __restrict__ C,
     const int32_t* __restrict__ Vv, const int64_t* __restrict__ off, int64_t n_m,
     const int32_t* __restrict__ cand, int S, int K, unsigned long long* __restrict__ cost,
@@ -287,43 +287,57 @@ __global__ __launch_bounds__(64 * kIrlpWaves, 4) void irlp_cost_kernel(
       acc.template totals<CB, G>(n, [&](int, uint64_t t) { best = t < best ? t : best; });
     } else {
       // Codes past 23 bits.  Many candidates: every coder in one pass over the
-      // samples (60 on 4,000 meshlets 126 us, 33 on 20,000 507; five passes of
-      // four coders 402 and 1,690).  Few: four coders a pass, whose registers
-      // leave the path above its waves (1 on 20,000 meshlets 64 us).
-      constexpr int kAt = CB >= 16 ? kCoders : 4;
-#pragma unroll 1
-      for (int j0 = 0; j0 < kCoders; j0 += kAt) {
-        uint64_t acc[kAt];
+      // samples, leading zeros counted in 32 bits (60 candidates on 4,000
+      // meshlets 119 us, 33 on 20,000 478; five passes of four coders 402 and
+      // 1,690).  Few, or more than 2^25 samples: four coders a pass, whose
+      // registers leave the path above its waves (1 on 20,000 meshlets 63 us).
+      auto value = [&](int32_t x, int32_t y, int32_t z, int32_t v) {
+        const int64_t s = (int64_t)n0 * x + (int64_t)n1 * y + (int64_t)n2 * z;
+        return zz64((int64_t)v - (K ? ((s + half) >> K) : s));
+      };
+      auto take = [&](int j, uint64_t acc) {
+        const uint64_t t = body_bits(j, coder_sum(j, group_sum<CB, G>(acc), n), n);
+        best = t < best ? t : best;
+      };
+      if (CB >= 16 && __all(n < (1u << 25))) {
+        uint64_t rice[kRiceK];
+        uint32_t zeros[kEgK];
 #pragma unroll
-        for (int q = 0; q < kAt; ++q) acc[q] = 0;
-        auto value = [&](int32_t x, int32_t y, int32_t z, int32_t v) {
-          const int64_t s = (int64_t)n0 * x + (int64_t)n1 * y + (int64_t)n2 * z;
-          return zz64((int64_t)v - (K ? ((s + half) >> K) : s));
+        for (int k = 0; k < kRiceK; ++k) rice[k] = 0;
+#pragma unroll
+        for (int k = 0; k < kEgK; ++k) zeros[k] = 0;
+        auto add = [&](uint64_t u) {
+#pragma unroll
+          for (int k = 0; k < kRiceK; ++k) rice[k] += u >> k;
+#pragma unroll
+          for (int k = 0; k < kEgK; ++k) zeros[k] += (uint32_t)__builtin_clzll(u + (1ull << k));
         };
-        if constexpr (kAt == kCoders) {
-          uint64_t i = slice;
-          if constexpr (SL == 1)   // two samples' scalar loads a trip
-            for (; i + 1 < n; i += 2) {
-              const int32_t x0 = a0[i], y0 = b0[i], z0 = c0[i], w0 = v0[i];
-              const int32_t x1 = a0[i + 1], y1 = b0[i + 1], z1 = c0[i + 1], w1 = v0[i + 1];
-              accumulate(value(x0, y0, z0, w0), acc);
-              accumulate(value(x1, y1, z1, w1), acc);
-            }
-          for (; i < n; i += SL) accumulate(value(a0[i], b0[i], c0[i], v0[i]), acc);
-        } else {
+        const uint32_t cnt = (uint32_t)n;
+        uint32_t i = slice;
+        for (; i + SL < cnt; i += 2 * SL) {   // two samples' loads a trip
+          const int32_t x0 = a0[i], y0 = b0[i], z0 = c0[i], w0 = v0[i];
+          const int32_t x1 = a0[i + SL], y1 = b0[i + SL], z1 = c0[i + SL], w1 = v0[i + SL];
+          add(value(x0, y0, z0, w0));
+          add(value(x1, y1, z1, w1));
+        }
+        if (i < cnt) add(value(a0[i], b0[i], c0[i], v0[i]));
+#pragma unroll
+        for (int k = 0; k < kRiceK; ++k) take(k, rice[k]);
+#pragma unroll
+        for (int k = 0; k < kEgK; ++k) take(kRiceK + k, zeros[k]);
+      } else {
+#pragma unroll 1
+        for (int j0 = 0; j0 < kCoders; j0 += 4) {
+          uint64_t acc[4] = {0, 0, 0, 0};
           for (uint64_t i = slice; i < n; i += SL) {
             const uint64_t u = value(a0[i], b0[i], c0[i], v0[i]);
 #pragma unroll
-            for (int q = 0; q < kAt; ++q)
+            for (int q = 0; q < 4; ++q)
               acc[q] += j0 < kRiceK ? u >> (j0 + q)
-                                     : (uint32_t)__builtin_clzll(u + (1ull << (j0 + q - kRiceK)));
+                                    : (uint32_t)__builtin_clzll(u + (1ull << (j0 + q - kRiceK)));
           }
-        }
 #pragma unroll
-        for (int q = 0; q < kAt; ++q) {
-          const uint64_t t =
-              body_bits(j0 + q, coder_sum(j0 + q, group_sum<CB, G>(acc[q]), n), n);
-          best = t < best ? t : best;
+          for (int q = 0; q < 4; ++q) take(j0 + q, acc[q]);
         }
       }
     }

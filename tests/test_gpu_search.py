@@ -131,3 +131,29 @@ def test_irls_leaves_degenerate_fits_to_the_host():
     assert search.IrlpCost(z, z, z, z, off).irls_l1() is None        # all zero
     assert search.IrlpCost(c + 7, c + 7, c, c, off).irls_l1() is None   # a = b
     assert search.IrlpCost(z[:0], z[:0], z[:0], z[:0], np.array([0, 0])).irls_l1() is None
+
+
+@pytest.mark.parametrize("n_streams", [1, 4, 5, 6143, 6144, 6145])
+@pytest.mark.parametrize("kind", ["small", "extreme"])
+def test_long_streams_among_short_ones(n_streams, kind):
+    """Streams on both sides of the 1,024 values from which a whole wave takes
+    one, anywhere among a wave's four, and of the line from which no workgroup
+    waits for them."""
+    from meshpress_amd.encoder import search
+    rng = np.random.default_rng(n_streams)
+    lens = rng.integers(0, 4, n_streams)
+    for i, n in ((0, 1024), (1, 1025), (n_streams // 2, 5000), (n_streams - 1, 1100)):
+        lens[min(i, n_streams - 1)] = n
+    off = np.concatenate(([0], np.cumsum(lens))).astype(np.int64)
+    vals = np.rint(rng.laplace(0, 20, off[-1])).astype(np.int32)
+    if kind == "extreme":
+        vals[::17] = -(1 << 31)
+        vals[3::29] = (1 << 31) - 1
+    want = coder_costs(zigzag(vals), off).astype(np.int64)
+    assert np.array_equal(search.stream_costs(vals, off), want)
+    tagk, bits = search.select_codes(vals, off)
+    rk, ek = want[:, :12].argmin(1), want[:, 12:].argmin(1)
+    rb, eb = want[:, :12].min(1), want[:, 12:].min(1)
+    rice = rb <= eb
+    assert np.array_equal(bits, np.where(rice, rb, eb))
+    assert np.array_equal(tagk, np.stack([np.where(rice, 1, 2), np.where(rice, rk, ek)], 1).astype(np.uint8))
