@@ -1,7 +1,7 @@
 // Encoder search kernels for gfx950.
 //
-//  * stream costs / selection: 16 lanes per residual stream; each lane folds
-//    its values into the 20 candidate body costs (Rice k = 0..11, Exp-Golomb
+//  * stream costs / selection: 16 lanes per residual stream (64 for long
+//    ones); each lane folds its values into the 20 candidate body costs (Rice k = 0..11, Exp-Golomb
 //    k = 0..7, residual_entropy.py:39-54 exact integer form), then a sum over
 //    the lanes and the tie-break of _pick_best_k
 //    (paradelta_v5_dup.py:159-171, paradelta_codec.py:131-146).
@@ -105,15 +105,15 @@ struct Costs32 {
       zeros[k] += (uint32_t)__builtin_clz(u + (1u << k)) + (uint32_t)__builtin_clz(v + (1u << k));
     slots += 2;
   }
-  // use(j, body cost) of n values over the lanes of group_sum<STEP, G>
-  template <int STEP, int G, class Use>
-  __device__ __forceinline__ void totals(uint64_t n, Use&& use) {
-    slots = group_sum<STEP, G>(slots);
+  // use(j, body cost) of n values; sum(x) adds x up over the lanes that hold them
+  template <class Sum, class Use>
+  __device__ __forceinline__ void totals(uint64_t n, Sum&& sum, Use&& use) {
+    slots = sum(slots);
 #pragma unroll
-    for (int k = 0; k < kRiceK; ++k) use(k, body_bits(k, group_sum<STEP, G>(rice[k]), n));
+    for (int k = 0; k < kRiceK; ++k) use(k, body_bits(k, sum(rice[k]), n));
 #pragma unroll
     for (int k = 0; k < kEgK; ++k) {
-      const uint32_t logs = slots * (uint32_t)(31 - k) - group_sum<STEP, G>(zeros[k]);
+      const uint32_t logs = slots * (uint32_t)(31 - k) - sum(zeros[k]);
       use(kRiceK + k, body_bits(kRiceK + k, 2ull * logs, n));
     }
   }
@@ -125,23 +125,31 @@ __device__ __forceinline__ bool fits_costs32(uint64_t n, uint64_t umax) {
   return n < (1u << 25) && umax < 0x80000000ull && (umax + 1) * n < 0x80000000ull;
 }
 
-constexpr int kStreamLanes = 16;   // the streams average 15 to 115 values
+// A mesh's streams average 15 to 115 values: four a wave, 16 lanes each.  Where
+// one of a wave's four is longer than kLongStream values all 64 lanes share a
+// stream: the wave takes the four in turn, or, up to kSpreadStreams streams,
+// whose waves do not fill the chip, the workgroup holds four waves for four
+// streams and each takes one (three of them end at once otherwise: 0.2 us at
+// 6,000 streams, 0.8 at 8,190).  Measured, against 16 lanes whatever the length
+// and a wave a stream in 64 bits: one stream of 4,000 values 18 us, 54 and 21;
+// 4,000 streams of 1,300 values 30, 89 and 40; 13,500 of them 108, 173 and 107;
+// 54,000 short streams 24, 25 and 137.
+constexpr int kStreamLanes = 16;
+constexpr int64_t kSpreadStreams = 6144, kLongStream = 1024;
 
-__global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restrict__ vals,
-                                                          const int64_t* __restrict__ off,
-                                                          int64_t n_streams,
-                                                          int64_t* __restrict__ costs,
-                                                          uint8_t* __restrict__ tagk,
-                                                          int64_t* __restrict__ best_bits) {
-  constexpr int G = kStreamLanes;
+// Stream s, the values [b, e), by a group of G lanes; s < 0: no stream, the
+// lanes take part in the sums with no values.
+template <int G>
+__device__ __forceinline__ void stream_cost(const int32_t* __restrict__ vals, int64_t s, int64_t b,
+                                            int64_t e, int64_t* __restrict__ costs,
+                                            uint8_t* __restrict__ tagk,
+                                            int64_t* __restrict__ best_bits) {
   const int lane = threadIdx.x % G;
-  const int64_t s = (int64_t)blockIdx.x * (256 / G) + threadIdx.x / G;
-  // lanes past the last stream take part in the sums with no values
-  const int64_t b = s < n_streams ? off[s] : 0, e = s < n_streams ? off[s + 1] : 0;
   const uint64_t n = (uint64_t)(e - b);
   uint32_t bits = 0;
   for (int64_t i = b + lane; i < e; i += G) bits |= zz32(vals[i]);
   const uint64_t umax = bits ? (2ull << (31 - __builtin_clz(bits))) - 1 : 0;
+  auto sum = [](auto v) { return group_sum<1, G>(v); };
   uint64_t tot[kCoders];
   if (__all(fits_costs32(n, umax))) {
     Costs32 acc;
@@ -151,16 +159,16 @@ __global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restr
       const uint32_t v = i + G < e ? zz32(vals[i + G]) : 0u;
       acc.add2(u, v);
     }
-    acc.totals<1, G>(n, [&](int j, uint64_t t) { tot[j] = t; });
+    acc.totals(n, sum, [&](int j, uint64_t t) { tot[j] = t; });
   } else {
     uint64_t acc[kCoders];
 #pragma unroll
     for (int j = 0; j < kCoders; ++j) acc[j] = 0;
     for (int64_t i = b + lane; i < e; i += G) accumulate(zz32(vals[i]), acc);
 #pragma unroll
-    for (int j = 0; j < kCoders; ++j) tot[j] = body_bits(j, coder_sum(j, group_sum<1, G>(acc[j]), n), n);
+    for (int j = 0; j < kCoders; ++j) tot[j] = body_bits(j, coder_sum(j, sum(acc[j]), n), n);
   }
-  if (lane == 0 && s < n_streams) {
+  if (lane == 0 && s >= 0) {
     if (costs) {
 #pragma unroll
       for (int j = 0; j < kCoders; ++j) costs[s * kCoders + j] = (int64_t)tot[j];
@@ -181,6 +189,40 @@ __global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restr
       if (best_bits) best_bits[s] = (int64_t)(rice ? rb : eb);
     }
   }
+}
+
+template <bool SPREAD>
+__global__ __launch_bounds__(256) void stream_cost_kernel(const int32_t* __restrict__ vals,
+                                                             const int64_t* __restrict__ off,
+                                                             int64_t n_streams,
+                                                             int64_t* __restrict__ costs,
+                                                             uint8_t* __restrict__ tagk,
+                                                             int64_t* __restrict__ best_bits) {
+  constexpr int G = kStreamLanes, W = 64 / G;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // the wave's first stream, and the lane's
+  const int64_t s0 = SPREAD ? W * (int64_t)blockIdx.x : W * (4 * (int64_t)blockIdx.x + wave);
+  const int64_t s = s0 + (threadIdx.x & 63) / G;
+  const bool some = s < n_streams;
+  const int64_t b = some ? off[s] : 0, e = some ? off[s + 1] : 0;
+  if (__builtin_expect(!__any(e - b > kLongStream), 1)) {
+    if (!SPREAD || wave == 0) stream_cost<G>(vals, some ? s : -1, b, e, costs, tagk, best_bits);
+    return;
+  }
+  const int64_t q1 = s0 + W < n_streams ? s0 + W : n_streams;
+#pragma unroll 1
+  for (int64_t q = SPREAD ? s0 + wave : s0; q < q1; q += SPREAD ? W : 1)
+    stream_cost<64>(vals, q, off[q], off[q + 1], costs, tagk, best_bits);
+}
+
+static hipError_t launch_streams(const int32_t* vals, const int64_t* off, int64_t n_streams,
+                                 int64_t* costs, uint8_t* tagk, int64_t* best_bits, hipStream_t st) {
+  const bool spread = n_streams <= kSpreadStreams;
+  const int64_t per = spread ? 4 : 16;
+  hipLaunchKernelGGL(spread ? stream_cost_kernel<true> : stream_cost_kernel<false>,
+                     dim3((unsigned)((n_streams + per - 1) / per)), dim3(256), 0, st, vals, off,
+                     n_streams, costs, tagk, best_bits);
+  return hipGetLastError();
 }
 
 // A wave's lanes are CB candidates x SL slices x MB meshlets (lane = (meshlet
@@ -284,7 +326,8 @@ __global__ __launch_bounds__(64 * kIrlpWaves) void irlp_cost_kernel(
           acc.add2(u, two ? v : 0u);
         }
       }
-      acc.template totals<CB, G>(n, [&](int, uint64_t t) { best = t < best ? t : best; });
+      acc.totals(n, [](auto v) { return group_sum<CB, G>(v); },
+                 [&](int, uint64_t t) { best = t < best ? t : best; });
     } else {
       // Codes past 23 bits.  Many candidates: every coder in one pass over the
       // samples, leading zeros counted in 32 bits (60 candidates on 4,000
@@ -541,10 +584,8 @@ extern "C" int stride_stream_costs(const int32_t* d_vals, const int64_t* d_off, 
   if (n_streams < 0 || (n_streams && (!d_vals || !d_off || !d_costs)))
     return set_error(STRIDE_E_ARG, "stride_stream_costs: null argument");
   if (n_streams == 0) return STRIDE_OK;
-  const int64_t blocks = (n_streams + 256 / kStreamLanes - 1) / (256 / kStreamLanes);
-  hipLaunchKernelGGL(stream_cost_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     (hipStream_t)stream, d_vals, d_off, n_streams, d_costs, nullptr, nullptr);
-  hipError_t e = hipGetLastError();
+  const hipError_t e =
+      launch_streams(d_vals, d_off, n_streams, d_costs, nullptr, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return set_error(STRIDE_E_HIP, hipGetErrorString(e));
   return STRIDE_OK;
 }
@@ -554,10 +595,8 @@ extern "C" int stride_select_codes(const int32_t* d_vals, const int64_t* d_off, 
   if (n_streams < 0 || (n_streams && (!d_vals || !d_off || !d_tagk)))
     return set_error(STRIDE_E_ARG, "stride_select_codes: null argument");
   if (n_streams == 0) return STRIDE_OK;
-  const int64_t blocks = (n_streams + 256 / kStreamLanes - 1) / (256 / kStreamLanes);
-  hipLaunchKernelGGL(stream_cost_kernel, dim3((unsigned)blocks), dim3(256), 0,
-                     (hipStream_t)stream, d_vals, d_off, n_streams, nullptr, d_tagk, d_bits);
-  hipError_t e = hipGetLastError();
+  const hipError_t e =
+      launch_streams(d_vals, d_off, n_streams, nullptr, d_tagk, d_bits, (hipStream_t)stream);
   if (e != hipSuccess) return set_error(STRIDE_E_HIP, hipGetErrorString(e));
   return STRIDE_OK;
 }
