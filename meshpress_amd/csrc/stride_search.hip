@@ -129,13 +129,13 @@ __device__ __forceinline__ bool fits_costs32(uint64_t n, uint64_t umax) {
 // one of a wave's four is longer than kLongStream values all 64 lanes share a
 // stream: the wave takes the four in turn, or, up to kSpreadStreams streams,
 // whose waves do not fill the chip, the workgroup holds four waves for four
-// streams and each takes one (three of them end at once otherwise: 0.2 us at
-// 6,000 streams, 0.8 at 8,190).  Measured, against 16 lanes whatever the length
+// streams and each takes one (three of them end at once otherwise: 0.5 us at
+// 8,190 streams, 1.7 at 12,288).  Measured, against 16 lanes whatever the length
 // and a wave a stream in 64 bits: one stream of 4,000 values 18 us, 54 and 21;
-// 4,000 streams of 1,300 values 30, 89 and 40; 13,500 of them 108, 173 and 107;
-// 54,000 short streams 24, 25 and 137.
+// 4,000 streams of 1,300 values 30, 89 and 40; 12,288 of them 66 (in turn 103),
+// 154 and 101; 13,500 in turn 105, 167 and 107; 54,000 short ones 24, 25, 137.
 constexpr int kStreamLanes = 16;
-constexpr int64_t kSpreadStreams = 6144, kLongStream = 1024;
+constexpr int64_t kSpreadStreams = 12288, kLongStream = 1024;
 
 // Stream s, the values [b, e), by a group of G lanes; s < 0: no stream, the
 // lanes take part in the sums with no values.

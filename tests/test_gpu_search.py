@@ -133,7 +133,7 @@ def test_irls_leaves_degenerate_fits_to_the_host():
     assert search.IrlpCost(z[:0], z[:0], z[:0], z[:0], np.array([0, 0])).irls_l1() is None
 
 
-@pytest.mark.parametrize("n_streams", [1, 4, 5, 6143, 6144, 6145])
+@pytest.mark.parametrize("n_streams", [1, 4, 5, 6145, 12287, 12288, 12289])
 @pytest.mark.parametrize("kind", ["small", "extreme"])
 def test_long_streams_among_short_ones(n_streams, kind):
     """Streams on both sides of the 1,024 values from which a whole wave takes
