@@ -1535,7 +1535,7 @@ STRIDE_DEV void scan_meshlet(const Src& src, uint32_t start, uint32_t end, const
   uint32_t st = 0, j = 0, lp = 0;
   for (;;) {
     if (j == lp) {
-      if (over()) { err = kScanErrOverrun; break; }
+      if (st && over()) { err = kScanErrOverrun; break; }   // after each strip
       if (st == ns) break;
       const uint32_t L = r.bits(16);
       ++st;
